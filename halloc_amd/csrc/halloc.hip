@@ -1029,9 +1029,10 @@ HA_DEV void free_rounds(const u64* off, const bool* act) {
 // Consecutive run rounds of hafree_batch (the rounds in the wave-uniform mask
 // F).  A run round frees blocks of one slab laid out as at most two runs of
 // consecutive k-chunk slots, one block per lane -- what one class group of
-// one wave allocates in one round.  Lane j holds round j's slab (sb), block
-// length (k) and run starts (sa, sbb); bit j of act/ina says whether this
-// lane frees a block in round j and whether it lies in the first run.
+// one wave allocates in one round.  The j-th ACTIVE lane holds round j's slab
+// (sb), block length (k) and run starts (sa, sbb): a lane the caller left
+// inactive holds nothing.  Bit j of act/ina says whether this lane frees a
+// block in round j and whether it lies in the first run.
 // Every round's nibbles are cleared before any result is awaited, then every
 // round's bits; then ONE counter decrement per slab for the total of its
 // rounds, each round's old count recovered in round order (what one-round
@@ -1040,35 +1041,47 @@ struct RunRounds {
   u32 sb, k, sa, sbb, sid, cid, act, ina;
 };
 
-// round j's wave-uniform values and this lane's place in it
+// round j's wave-uniform values (lane l holds them) and this lane's place in it
 struct RunRound {
   u32 sb, k, st, ich;
   bool act, ina;
   u64 Am, Bm;
 };
-HA_DEV RunRound run_round(const RunRounds& r, u32 j) {
+HA_DEV RunRound run_round(const RunRounds& r, u32 j, u32 l) {
   RunRound x;
-  x.sb = rdl(r.sb, j);
-  x.k = rdl(r.k, j);
+  x.sb = rdl(r.sb, l);
+  x.k = rdl(r.k, l);
   x.act = (r.act >> j) & 1;
   x.ina = (r.ina >> j) & 1;
   x.Am = ballot(x.act && x.ina);
   x.Bm = ballot(x.act && !x.ina);
-  x.st = x.ina ? rdl(r.sa, j) : rdl(r.sbb, j);
+  x.st = x.ina ? rdl(r.sa, l) : rdl(r.sbb, l);
   x.ich = x.st + lane_id() * x.k;
   return x;
 }
 
+// the lane that holds the next round (a walk over the active lanes)
+HA_DEV u32 next_lane(u64& walk) {
+  const u32 l = (u32)__builtin_ctzll(walk);
+  walk &= walk - 1;
+  return l;
+}
+
 HA_DEV void free_runs(u32 F, RunRounds r) {
   const u32 me = lane_id();
+  const u64 lanes = ballot(true);
+  const u32 jme = (u32)__builtin_popcountll(lanes & ((1ull << me) - 1));  // the round this lane holds
+  const u32 nr = 32u - (u32)__builtin_clz(F);  // rounds up to the last in F: one active lane each
   // every round's nibbles, no result awaited (o is indexed by the
   // wave-uniform round: it stays in registers)
   u64 o[MAXB];
+  u64 walk = lanes;
 #pragma nounroll
-  for (u32 j = 0; j < MAXB; ++j) {
+  for (u32 j = 0; j < nr; ++j) {
+    const u32 l = next_lane(walk);
     u64 v = 0;
     if ((F >> j) & 1) {
-      const RunRound x = run_round(r, j);
+      const RunRound x = run_round(r, j, l);
       u32 wn, inn;
       u64 un;
       run_word_nibs(x.ina ? x.Am : x.Bm, me, x.st, x.k, 0xFull, wn, un, inn);
@@ -1077,11 +1090,13 @@ HA_DEV void free_runs(u32 F, RunRounds r) {
     o[j] = v;
   }
   // then every round's bits and change
-  u32 rch = 0;  // lane j: chunks freed in round j
+  u32 rch = 0;  // the round's lane: chunks freed in the round
+  walk = lanes;
 #pragma nounroll
-  for (u32 j = 0; j < MAXB; ++j) {
+  for (u32 j = 0; j < nr; ++j) {
+    const u32 l = next_lane(walk);
     if (!((F >> j) & 1)) continue;
-    const RunRound x = run_round(r, j);
+    const RunRound x = run_round(r, j, l);
     const u64 myseg = x.ina ? x.Am : x.Bm;
     u32 wn, inn;
     u64 un;
@@ -1107,12 +1122,12 @@ HA_DEV void free_runs(u32 F, RunRounds r) {
 #pragma unroll
       for (u32 b = 0; b < 4; ++b) change += (u32)__builtin_popcountll(ballot((nch >> b) & 1)) << b;
     }
-    rch = wrl(change, j, rch);
+    rch = wrl(change, l, rch);
   }
   const u32 rsb = r.sb, rsid = r.sid, rcid = r.cid;
   // one decrement per slab, by the lane of its first round; pre = the
   // changes of the slab's earlier rounds
-  const bool inF = me < MAXB && ((F >> me) & 1) && rch != 0;
+  const bool inF = jme < nr && ((F >> jme) & 1) && rch != 0;
   u32 pre = 0, tot = 0, ldr = 0;
   for (u64 rem = ballot(inF); rem;) {
     const u32 l = (u32)__builtin_ctzll(rem);
@@ -1357,13 +1372,20 @@ HA_API void hafree_batch(void* const* ptrs, int cnt) {
   // see free_rounds: one release per call for a cached arena
   if (ha_p.cached_arena) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
   const u32 me = lane_id();
-  // every round's slab, where all its blocks lie in one (lane j: round j's)
+  // every round's slab, where all its blocks lie in one (the j-th active lane
+  // holds round j's; with fewer active lanes than rounds, every round goes
+  // through the one-round path)
+  const u64 lanes = ballot(true);
+  const u32 jme = (u32)__builtin_popcountll(lanes & ((1ull << me) - 1));
+  const bool held = (u32)__builtin_popcountll(lanes) >= R;
   u32 ino[MAXB];  // in-slab offsets
   u32 actm = 0, single = 0, rsb = 0;
+  u64 walk = lanes;
 #pragma nounroll
   for (u32 j = 0; j < MAXB; ++j) {
     ino[j] = 0;
     if (j >= R) continue;
+    const u32 l = held ? next_lane(walk) : 0u;
     void* p = j < c ? ptrs[j] : nullptr;
     const u64 off = (u64)((char*)p - ha_p.arena);
     const bool act = p && off < ha_p.arena_bytes;
@@ -1371,16 +1393,16 @@ HA_API void hafree_batch(void* const* ptrs, int cnt) {
     ino[j] = (u32)(off & (ha_p.sb_sz - 1));
     actm |= (u32)act << j;
     const u64 A = ballot(act);
-    if (!A) continue;
+    if (!A || !held) continue;
     const u32 sb0 = rdl(sb, (u32)__builtin_ctzll(A));
     if (ballot(act && sb == sb0) == A) {
       single |= 1u << j;
-      rsb = wrl(sb0, j, rsb);
+      rsb = wrl(sb0, l, rsb);
     }
   }
   // their descriptors: one load per round
   u32 rcs = 0, rsid = SZ_NONE, rcid = SZ_NONE;
-  if (me < MAXB && ((single >> me) & 1)) {
+  if (jme < MAXB && ((single >> jme) & 1)) {
     Desc* d = ha_p.desc + rsb;
     rcs = ld32(&d->chunk_sz);
     rsid = ld32(&d->size_id);
@@ -1388,10 +1410,13 @@ HA_API void hafree_batch(void* const* ptrs, int cnt) {
   }
   // which of them are run rounds
   u32 fast = 0, inam = 0, rk = 0, rsa = 0, rsbb = 0;
+  walk = lanes;
 #pragma nounroll
   for (u32 j = 0; j < MAXB; ++j) {
+    if (j >= R || !held) continue;
+    const u32 l = next_lane(walk);
     if (!((single >> j) & 1)) continue;
-    const u32 cs = rdl(rcs, j), sid = rdl(rsid, j);
+    const u32 cs = rdl(rcs, l), sid = rdl(rsid, l);
     if (cs == 0 || sid >= NSIZES) continue;
     const bool act = (actm >> j) & 1;
     const u32 ich = act ? chunk_div(ino[j], cs) : 0u;
@@ -1412,9 +1437,9 @@ HA_API void hafree_batch(void* const* ptrs, int cnt) {
     if ((Am | Bm) == A && ((sa | sbb) & (k - 1)) == 0) {
       fast |= 1u << j;
       inam |= (u32)ina << j;
-      rk = wrl(k, j, rk);
-      rsa = wrl(sa, j, rsa);
-      rsbb = wrl(sbb, j, rsbb);
+      rk = wrl(k, l, rk);
+      rsa = wrl(sa, l, rsa);
+      rsbb = wrl(sbb, l, rsbb);
     }
   }
   // round order: runs of run rounds together, the others one by one

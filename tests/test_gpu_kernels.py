@@ -43,3 +43,41 @@ def test_null_check_counts_the_nulls_held(heap, test, n, bs, nallocs, period, gr
     assert r["checks_failed"] == r["nulls"]
     assert r["failed_try"] == (0 if r["nulls"] else -1)
     assert r["mallocs"] == r["frees"]
+
+
+# lanes that take part in a batched call: a wave whose low lanes are inactive
+# (the per-round values must not be kept in lanes 0..15), fewer lanes than
+# rounds, every other lane, one lane
+PARTIAL_WAVES = {"high": range(16, 64), "few": range(40, 47), "odd": range(1, 64, 2), "mixed": [2, 3, 9, 11, 14, 30, 31, 55],
+                 "last": [63], "sixteen": range(48, 64)}
+
+
+def partial_batch_ops(lanes, sizes=(16, 48, 128, 24, 700, 3072), cnt=16):
+    """Every size: two batches of cnt blocks per lane, the first freed, then freed again (nothing happens),
+    then the second freed together with a third batch's allocation by the other lanes."""
+    rows = []
+    for sz in sizes:
+        r = len(rows)
+        for kind in (1, 1, 3, 2, 2):
+            row = np.zeros((64, 4), dtype=np.uint32)
+            for l in lanes:
+                src = {3: r, 2: r if len(rows) == r + 3 else r + 1}.get(kind, 0)
+                row[l] = (1, sz, cnt - l % 3, 0) if kind == 1 else (kind, src * 64 + l, 0, 0)
+            rows.append(row)
+    return np.stack(rows)
+
+
+@pytest.mark.parametrize("which", sorted(PARTIAL_WAVES))
+def test_batched_free_of_a_partial_wave(heap, which):
+    # bit-exact against the host model, and the heap empty at the end
+    from oracle import model as M
+    print(f"[gpu] batched free, lanes {which}", flush=True)
+    opts = heap(H.HallocOpts(memory=256 << 20, sb_sz_sh=21, nheads=1))
+    ops = partial_batch_ops(PARTIAL_WAVES[which])
+    recs, xcc = H.Halloc.replay_batch(ops)
+    m = M.ModelHeap(M.make_opts(memory=opts.memory, sb_sz_sh=opts.sb_sz_sh, nheads=1, hash_mode=1))
+    want = m.replay_batch(ops, xcc % 1)
+    assert (recs == want).all()
+    d = H.Halloc.dump()
+    assert (d == m.dump()).all()
+    assert ((d[:H.Halloc.geometry()["nsbs"]] >> np.uint64(32)) == 0).all()
