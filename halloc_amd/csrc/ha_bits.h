@@ -15,36 +15,34 @@ namespace ha {
 using u32 = uint32_t;
 using u64 = uint64_t;
 
-// bit i of x moves to bit f*i (x holds at most 64/f meaningful bits)
-HA_HD inline u64 spread_bits(u64 x, u32 f) {
+// bit i of x moves to bit f*i (x holds at most 64/f meaningful bits).  Each
+// 32-bit half is spread by itself: the shift-or-mask steps are one
+// instruction each in 32 bits, and two or more in 64.
+HA_HD inline u32 spread_half(u32 x, u32 f) {
   switch (f) {
-    case 1:
-      return x;
     case 2:
-      x &= 0xffffffffull;
-      x = (x | x << 16) & 0x0000FFFF0000FFFFull;
-      x = (x | x << 8) & 0x00FF00FF00FF00FFull;
-      x = (x | x << 4) & 0x0F0F0F0F0F0F0F0Full;
-      x = (x | x << 2) & 0x3333333333333333ull;
-      return (x | x << 1) & 0x5555555555555555ull;
+      x = (x | x << 8) & 0x00FF00FFu;
+      x = (x | x << 4) & 0x0F0F0F0Fu;
+      x = (x | x << 2) & 0x33333333u;
+      return (x | x << 1) & 0x55555555u;
     case 4:
-      x &= 0xffffull;
-      x = (x | x << 24) & 0x000000FF000000FFull;
-      x = (x | x << 12) & 0x000F000F000F000Full;
-      x = (x | x << 6) & 0x0303030303030303ull;
-      return (x | x << 3) & 0x1111111111111111ull;
+      x = (x | x << 12) & 0x000F000Fu;
+      x = (x | x << 6) & 0x03030303u;
+      return (x | x << 3) & 0x11111111u;
     case 8:
-      x &= 0xffull;
-      x = (x | x << 28) & 0x0000000F0000000Full;
-      x = (x | x << 14) & 0x0003000300030003ull;
-      return (x | x << 7) & 0x0101010101010101ull;
+      x = (x | x << 14) & 0x00030003u;
+      return (x | x << 7) & 0x01010101u;
     case 16:
-      return (x & 1) | ((x & 2) << 15) | ((x & 4) << 30) | ((x & 8) << 45);
-    case 32:
-      return (x & 1) | ((x & 2) << 31);
-    default:
-      return 0;
+      return (x | x << 15) & 0x00010001u;
+    default:  // 32
+      return x;
   }
+}
+HA_HD inline u64 spread_bits(u64 x, u32 f) {
+  if (f == 1) return x;
+  if (f > 32) return 0;
+  const u32 h = 32 / f, m = h >= 32 ? ~0u : (1u << h) - 1;
+  return (u64)spread_half((u32)(x >> h) & m, f) << 32 | spread_half((u32)x & m, f);
 }
 
 // A run of 64 k-chunk slots starts at chunk s (slot of lane l = s + l*k,
@@ -54,37 +52,38 @@ HA_HD inline u64 spread_bits(u64 x, u32 f) {
 // index of the word holding me's slot, the union of B-lanes' fields inside that
 // word, and the lowest B-lane in that word (64 if none).
 //   bit array:    64 chunks per word, field = k one-bits
-//   nibble array: 16 chunks per word, field = 4-bit value `val` at the slot start
+//   nibble array: 16 chunks per word, field = 4-bit value `val` (15 or a power
+//                 of two) at the slot start
+// With j = the slot's place in its word, the word holds the lanes me - j on:
+// B shifted there, cut to the word's slots, is the word's lanes slot by slot,
+// and spreading them gives the union already in place.
+HA_HD inline u64 word_lanes(u64 B, int d) { return d >= 0 ? B >> (d & 63) : B << (-d & 63); }
 HA_HD inline void run_word_bits(u64 B, u32 me, u32 s, u32 k, u32& word, u64& uni, u32& issuer) {
-  u32 c = s + me * k;
+  const u32 c = s + me * k;
   word = c >> 6;
   const u32 ks = (u32)__builtin_ctz(k);
-  int lo_u = (int)(word << 6) - (int)s;
-  u32 lo = lo_u <= 0 ? 0u : (u32)lo_u >> ks;
-  u32 hi = (u32)(lo_u + 63) >> ks;
-  hi = hi > 63 ? 63 : hi;
-  u32 n = hi - lo + 1;
-  u64 m = n >= 64 ? ~0ull : ((1ull << n) - 1);
-  u64 sub = (B >> lo) & m;
-  u32 sh = s + lo * k - (word << 6);
-  uni = (spread_bits(sub, k) * ((1ull << k) - 1)) << sh;
-  issuer = sub ? lo + (u32)__builtin_ctzll(sub) : 64u;
+  const int d = (int)me - (int)((c & 63u) >> ks);  // lane of the word's first slot
+  const u64 x = word_lanes(B, d);
+  if (k == 1) {
+    uni = x;
+    issuer = x ? (u32)(d + (int)__builtin_ctzll(x)) : 64u;
+  } else {
+    const u32 y = k == 2 ? (u32)x : (u32)x & ((1u << (64u >> ks)) - 1);
+    const u64 t = spread_bits(y, k);
+    uni = (t << k) - t;  // every slot's first bit widened to k ones
+    issuer = y ? (u32)(d + (int)__builtin_ctz(y)) : 64u;
+  }
 }
 HA_HD inline void run_word_nibs(u64 B, u32 me, u32 s, u32 k, u64 val, u32& word, u64& uni,
                                               u32& issuer) {
-  u32 c = s + me * k;
+  const u32 c = s + me * k;
   word = c >> 4;
   const u32 ks = (u32)__builtin_ctz(k);
-  int lo_u = (int)(word << 4) - (int)s;
-  u32 lo = lo_u <= 0 ? 0u : (u32)lo_u >> ks;
-  u32 hi = (u32)(lo_u + 15) >> ks;
-  hi = hi > 63 ? 63 : hi;
-  u32 n = hi - lo + 1;
-  u64 m = n >= 64 ? ~0ull : ((1ull << n) - 1);
-  u64 sub = (B >> lo) & m;
-  u32 sh = s + lo * k - (word << 4);
-  uni = (spread_bits(sub, 4 * k) * val) << (4 * sh);
-  issuer = sub ? lo + (u32)__builtin_ctzll(sub) : 64u;
+  const int d = (int)me - (int)((c & 15u) >> ks);
+  const u32 y = (u32)word_lanes(B, d) & ((1u << (16u >> ks)) - 1);
+  const u64 t = spread_bits(y, 4 * k);
+  uni = val == 15 ? (t << 4) - t : t << (u32)__builtin_ctzll(val);
+  issuer = y ? (u32)(d + (int)__builtin_ctz(y)) : 64u;
 }
 
 // ----------------------------------------------------------- unit fields

@@ -70,7 +70,9 @@ struct SizeInfo {
   u32 pad[2];
 };
 
-struct Desc {
+// the size id and the chunk id share an aligned 64-bit word: a free reads both
+// in one load
+struct alignas(16) Desc {
   u32 size_id, chunk_id, chunk_sz, is_head;
 };
 

@@ -47,6 +47,7 @@ HA_DEV u64 rdl64(u64 v, u32 lane) {
   return ((u64)rdl((u32)(v >> 32), lane) << 32) | rdl((u32)v, lane);
 }
 HA_DEV u32 rfl(u32 v) { return (u32)__builtin_amdgcn_readfirstlane((int)v); }
+HA_DEV u64 rfl64(u64 v) { return ((u64)rfl((u32)(v >> 32)) << 32) | rfl((u32)v); }
 // v with lane `lane` replaced by the wave-uniform x
 HA_DEV u32 wrl(u32 x, u32 lane, u32 v) { return lane_id() == lane ? x : v; }
 HA_DEV u64 shfl64(u64 v, u32 src) {
@@ -58,26 +59,42 @@ HA_DEV u64 shfl64(u64 v, u32 src) {
 HA_DEV u32 xcc_id() { return __builtin_amdgcn_s_getreg((20) | (0 << 6) | ((4 - 1) << 11)); }
 // HW_ID bits 8..15: the wave's CU, shader array and shader engine
 HA_DEV u32 cu_bits() { return __builtin_amdgcn_s_getreg((4) | (8 << 6) | ((8 - 1) << 11)); }
+// The parameter block, read where it is used: the volatile asm keeps the
+// compiler from loading parameters ahead, in the code every wave runs, and
+// holding them there.  Held, they overflow the 102 SGPRs: of the 734 vector
+// instructions of a 16 B malloc and free 358 were spills to VGPR lanes and
+// their reloads.
+HA_DEV const Params& params() {
+  typedef const __attribute__((address_space(4))) Params* cptr;
+  cptr p = (cptr)(uintptr_t)&ha_p;
+  __asm__ volatile("" : "+s"(p));
+  return *(const Params*)p;
+}
 // The head set a wave would use with every set in use: its XCD's, and with
 // more than 8 sets (a multiple of 8), one of the XCD's nheads / 8 sets picked
 // by the wave's CU.
-HA_DEV u32 head_set() {
-  const u32 x = xcc_id(), n = ha_p.nheads;
-  if (n <= 8) return mod_by(x, n, ha_p.nh_m);
-  return x + 8u * mod_by(cu_bits(), n / 8u, ha_p.nh8_m);  // x < 8: already below n
+HA_DEV u32 head_set(const Params& P) {
+  const u32 x = xcc_id(), n = P.nheads;
+  if (n <= 8) return mod_by(x, n, P.nh_m);
+  return x + 8u * mod_by(cu_bits(), n / 8u, P.nh8_m);  // x < 8: already below n
 }
 // Set `full` (< nheads) folded onto the first s sets (s = nheads, or a power
 // of two below it): the XCD part keeps its low bits, the CU part its low bits.
-HA_DEV u32 fold_set(u32 full, u32 s) {
-  if (s >= ha_p.nheads) return full;
+HA_DEV u32 fold_set(const Params& P, u32 full, u32 s) {
+  if (s >= P.nheads) return full;
   if (s <= 8) return full & (s - 1);
   return (full & 7u) + 8u * ((full >> 3) & (s / 8u - 1));
 }
 // The sets in use now, read through the scalar cache: a stale value (the
 // spread only shrinks while a kernel runs) still names valid sets.
-HA_DEV u32 spread_cached() {
-  if (ha_p.fixed_sets) return ha_p.nheads;
-  return *(const __attribute__((address_space(4))) u32*)(uintptr_t)ha_p.spread;
+HA_DEV u32 spread_cached(const Params& P) {
+  if (P.fixed_sets) return P.nheads;
+  return *(const __attribute__((address_space(4))) u32*)(uintptr_t)P.spread;
+}
+// the set of the calling wave's mallocs
+HA_DEV u32 wave_set() {
+  const Params& P = params();
+  return rfl(fold_set(P, head_set(P), spread_cached(P)));
 }
 
 // ------------------------------------------------ agent-scope atomic helpers
@@ -92,15 +109,25 @@ HA_DEV u64 ld64(u64* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, HA_SCOPE
 HA_DEV u32 ld32(u32* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, HA_SCOPE); }
 HA_DEV void st32(u32* p, u32 v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, HA_SCOPE); }
 
-HA_DEV u64* ctr_of(u32 sb) { return ha_p.ctr + (u64)sb * CTR_STRIDE; }
+HA_DEV u64* ctr_of(const Params& P, u32 sb) { return P.ctr + (u64)sb * CTR_STRIDE; }
+// a slab's first word of the bit and nibble arrays, and its first byte
+// (bit_words = sb_sz / 1024 and nib_words = sb_sz / 256 words per slab)
+HA_DEV u64* bits_of(const Params& P, u32 sb) { return P.bits + ((u64)sb << (P.sb_sz_sh - 10)); }
+HA_DEV u64* nibs_of(const Params& P, u32 sb) { return P.nibs + ((u64)sb << (P.sb_sz_sh - 8)); }
+HA_DEV char* slab_of(const Params& P, u32 sb) { return P.arena + ((u64)sb << P.sb_sz_sh); }
 HA_DEV u32* hot(u32* base, u32 ihead, u32 sid) { return base + (ihead * NSIZES + sid) * HOT_STRIDE; }
-HA_DEV u64* set_words(u32 set) { return ha_p.sets + (u64)set * ha_p.nsw; }
+HA_DEV u64* set_words(const Params& P, u32 set) { return P.sets + (u64)set * P.nsw; }
 
 // ----------------------------------------------------- single-lane slow path
 // Everything below until malloc_group runs on exactly one lane of a wave.
 
+// loads of the one active lane, wave-uniform: the slow path's branches and
+// addresses stay scalar instead of nesting exec masks in SGPR pairs
+HA_DEV u32 ul32(u32* p) { return rfl(ld32(p)); }
+HA_DEV u64 ul64(u64* p) { return rfl64(ld64(p)); }
+
 HA_DEV bool try_lock(u32* m) {
-  bool ok = a_xchg32(m, 1u) == 0;
+  bool ok = rfl(a_xchg32(m, 1u)) == 0;
   if (ok) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   return ok;
 }
@@ -112,17 +139,17 @@ HA_DEV void unlock(u32* m) {
   st32(m, 0u);
 }
 
-HA_DEV void set_add(u32 set, u32 sb) { a_or(set_words(set) + sb / 64, 1ull << (sb % 64)); }
-HA_DEV void set_remove(u32 set, u32 sb) { a_and(set_words(set) + sb / 64, ~(1ull << (sb % 64))); }
+HA_DEV void set_add(const Params& P, u32 set, u32 sb) { a_or(set_words(P, set) + sb / 64, 1ull << (sb % 64)); }
+HA_DEV void set_remove(const Params& P, u32 set, u32 sb) { a_and(set_words(P, set) + sb / 64, ~(1ull << (sb % 64))); }
 // first-fit claim over every word holding a slab (src/sbset.cuh:5-35)
-HA_DEV u32 set_pop(u32 set) {
-  u64* w = set_words(set);
-  for (u32 i = 0; i < ha_p.nsw; ++i) {
-    u64 word = ld64(w + i);
+HA_DEV u32 set_pop(const Params& P, u32 set) {
+  u64* w = set_words(P, set);
+  for (u32 i = 0; i < P.nsw; ++i) {
+    u64 word = ul64(w + i);
     while (word) {
       u32 b = (u32)__builtin_ctzll(word);
       u64 m = 1ull << b;
-      if (a_and(w + i, ~m) & m) return i * 64 + b;
+      if (rfl64(a_and(w + i, ~m)) & m) return i * 64 + b;
       word &= ~m;
     }
   }
@@ -130,57 +157,59 @@ HA_DEV u32 set_pop(u32 set) {
 }
 
 // sb_try_mark_free (src/slab.cuh:89-113); caller holds sb_lock[sb]
-HA_DEV void try_mark_free(u32 sb, u32 size_id, u32 chunk_id, bool from_head) {
-  Desc* d = ha_p.desc + sb;
-  if (ld32(&d->is_head) || chunk_id == SZ_NONE) return;
+HA_DEV void try_mark_free(const Params& P, u32 sb, u32 size_id, u32 chunk_id, bool from_head) {
+  Desc* d = P.desc + sb;
+  if (ul32(&d->is_head) || chunk_id == SZ_NONE) return;
   u64 delta = ctr_chunk_delta(chunk_id), old2;
-  u64* c = ctr_of(sb);
+  u64* c = ctr_of(P, sb);
   do {
-    u64 old = a_add(c, delta);
+    u64 old = rfl64(a_add(c, delta));
     if (ctr_count(old) == 0) {
       st32(&d->size_id, SZ_NONE);
       st32(&d->chunk_id, SZ_NONE);
       st32(&d->chunk_sz, 0);
-      set_add(0, sb);
-      a_add32(ha_p.free_ep, 1u);
-      set_remove(set_sparse(chunk_id), sb);
+      set_add(P, 0, sb);
+      a_add32(P.free_ep, 1u);
+      set_remove(P, set_sparse(chunk_id), sb);
       if (size_id != SZ_NONE) {
-        set_remove(set_roomy(size_id), sb);
-        set_remove(set_busy(size_id), sb);
+        set_remove(P, set_roomy(size_id), sb);
+        set_remove(P, set_busy(size_id), sb);
       }
       return;
     }
-    old2 = a_sub(c, delta);
+    old2 = rfl64(a_sub(c, delta));
   } while (ctr_count(old2) == 0);
   if (from_head && size_id != SZ_NONE) {
-    u32 cls = sb_class(ctr_count(old2), ha_p.si[size_id]);
-    if (cls != CLS_FREE) set_add(class_set(cls, size_id, chunk_id), sb);
+    u32 cls = sb_class(ctr_count(old2), P.si[size_id]);
+    if (cls != CLS_FREE) set_add(P, class_set(cls, size_id, chunk_id), sb);
   }
 }
 
 // count transitions after a decrement (src/slab.cuh:176-221): `old` is the
 // counter before the decrement of `change` chunks
 HA_DEV void ctr_transitions(u32 sb, u64 old, u32 change) {
+  sb = rfl(sb), old = rfl64(old), change = rfl(change);
   if (ctr_is_head(old)) return;
-  Desc* d = ha_p.desc + sb;
-  u32 size_id = ld32(&d->size_id), chunk_id = ld32(&d->chunk_id);
+  const Params& P = params();
+  Desc* d = P.desc + sb;
+  u32 size_id = ul32(&d->size_id), chunk_id = ul32(&d->chunk_id);
   if (size_id == SZ_NONE || chunk_id == SZ_NONE) return;
   u32 oc = ctr_count(old), nc = oc - change;
-  const SizeInfo& s = ha_p.si[size_id];
+  const SizeInfo& s = P.si[size_id];
   u32 co = sb_class(oc, s), cn = sb_class(nc, s);
   if (co == cn) return;
   if (cn == CLS_FREE) {
     if (ctr_chunk(old) != CTR_CHUNK_NONE) {
-      u32* l = ha_p.sb_lock + sb;
+      u32* l = P.sb_lock + sb;
       lock(l);
-      size_id = ld32(&d->size_id);
-      chunk_id = ld32(&d->chunk_id);
-      try_mark_free(sb, size_id, chunk_id, false);
+      size_id = ul32(&d->size_id);
+      chunk_id = ul32(&d->chunk_id);
+      try_mark_free(P, sb, size_id, chunk_id, false);
       unlock(l);
     }
   } else {
-    set_add(class_set(cn, size_id, chunk_id), sb);
-    if (co != CLS_FREE) set_remove(class_set(co, size_id, chunk_id), sb);
+    set_add(P, class_set(cn, size_id, chunk_id), sb);
+    if (co != CLS_FREE) set_remove(P, class_set(co, size_id, chunk_id), sb);
   }
 }
 
@@ -188,42 +217,42 @@ HA_DEV void ctr_transitions(u32 sb, u64 old, u32 change) {
 // drop one head reference (detach_head, src/slab.cuh:227-255); the last one
 // files the slab by its count.  Caller holds sb_lock[sb].  True if the slab
 // became free.
-HA_DEV bool detach_head(u32 sb) {
-  Desc* d = ha_p.desc + sb;
-  const u32 refs = ld32(&d->is_head) - 1;
+HA_DEV bool detach_head(const Params& P, u32 sb) {
+  Desc* d = P.desc + sb;
+  const u32 refs = ul32(&d->is_head) - 1;
   st32(&d->is_head, refs);
-  u64 old = a_sub(ctr_of(sb), CTR_HEAD);
+  u64 old = rfl64(a_sub(ctr_of(P, sb), CTR_HEAD));
   if (refs) return false;
   u32 count = ctr_count(old);
-  u32 size_id = ld32(&d->size_id), chunk_id = ld32(&d->chunk_id);
+  u32 size_id = ul32(&d->size_id), chunk_id = ul32(&d->chunk_id);
   if (size_id == SZ_NONE) return false;
-  u32 cls = sb_class(count, ha_p.si[size_id]);
+  u32 cls = sb_class(count, P.si[size_id]);
   if (cls == CLS_FREE) {
-    try_mark_free(sb, size_id, chunk_id, true);
-    return ld32(&d->chunk_id) == SZ_NONE;
+    try_mark_free(P, sb, size_id, chunk_id, true);
+    return ul32(&d->chunk_id) == SZ_NONE;
   }
-  set_add(class_set(cls, size_id, chunk_id), sb);
+  set_add(P, class_set(cls, size_id, chunk_id), sb);
   return false;
 }
 
 // Shares the head of another XCD's pair of the same class if it has room.
 // Caller holds the head lock of (ihead, size_id).
-HA_DEV u32 share_head(u32 ihead, u32 size_id, u32 chunk_id) {
-  const SizeInfo& s = ha_p.si[size_id];
-  for (u32 ih = 0; ih < ha_p.nheads; ++ih) {
+HA_DEV u32 share_head(const Params& P, u32 ihead, u32 size_id, u32 chunk_id) {
+  const SizeInfo& s = P.si[size_id];
+  for (u32 ih = 0; ih < P.nheads; ++ih) {
     if (ih == ihead) continue;
-    u32 w = ld32(hot(ha_p.head, ih, size_id));
+    u32 w = ul32(hot(P.head, ih, size_id));
     if (w == SB_NONE) continue;
     u32 sb = w & ~HEAD_EXT;
-    if (ctr_count(ld64(ctr_of(sb))) >= head_limit(w, s)) continue;
-    Desc* d = ha_p.desc + sb;
-    u32* l = ha_p.sb_lock + sb;
+    if (ctr_count(ul64(ctr_of(P, sb))) >= head_limit(w, s)) continue;
+    Desc* d = P.desc + sb;
+    u32* l = P.sb_lock + sb;
     lock(l);
-    u32 refs = ld32(&d->is_head);
-    bool ok = refs > 0 && refs < 255 && ld32(&d->size_id) == size_id && ctr_chunk(ld64(ctr_of(sb))) == chunk_id;
+    u32 refs = ul32(&d->is_head);
+    bool ok = refs > 0 && refs < 255 && ul32(&d->size_id) == size_id && ctr_chunk(ul64(ctr_of(P, sb))) == chunk_id;
     if (ok) {
       st32(&d->is_head, refs + 1);
-      a_add(ctr_of(sb), CTR_HEAD);
+      a_add(ctr_of(P, sb), CTR_HEAD);
     }
     unlock(l);
     if (ok) return w;
@@ -239,33 +268,33 @@ HA_DEV u32 share_head(u32 ihead, u32 size_id, u32 chunk_id) {
 // that never took a head holds none, so only the classes seen are visited
 // (in the same set-major order): with one class the idle search costs
 // nothing.
-HA_DEV bool steal_idle_head(u32 ihead, u32 size_id, bool other_idle = false) {
-  const u32 nh = ha_p.nheads;
-  const u32 sp = ha_p.fixed_sets ? nh : ld32(ha_p.spread);
-  u32 cls = ha_p.fixed_sets ? (1u << NSIZES) - 1 : ld32(ha_p.class_seen) & ((1u << NSIZES) - 1);
+HA_DEV bool steal_idle_head(const Params& P, u32 ihead, u32 size_id, bool other_idle = false) {
+  const u32 nh = P.nheads;
+  const u32 sp = P.fixed_sets ? nh : ul32(P.spread);
+  u32 cls = P.fixed_sets ? (1u << NSIZES) - 1 : ul32(P.class_seen) & ((1u << NSIZES) - 1);
   if (other_idle) cls &= ~(1u << size_id);
   if (!cls) return false;
   for (u32 ih = 0; ih < nh; ++ih) {
     for (u32 rem = cls; rem; rem &= rem - 1) {
       const u32 c = (u32)__builtin_ctz(rem);
       if (ih == ihead && c == size_id) continue;
-      u32* lp = hot(ha_p.head_lock, ih, c);
+      u32* lp = hot(P.head_lock, ih, c);
       for (int which = 0; which < 2; ++which) {
         if (other_idle && which == 1 && ih < sp) continue;
-        u32* wp = hot(which == 0 ? ha_p.cached : ha_p.head, ih, c);
-        u32 w = ld32(wp);
+        u32* wp = hot(which == 0 ? P.cached : P.head, ih, c);
+        u32 w = ul32(wp);
         if (w == SB_NONE) continue;
         u32 sb = w & ~HEAD_EXT;
-        if (ctr_count(ld64(ctr_of(sb))) != 0) continue;
+        if (ctr_count(ul64(ctr_of(P, sb))) != 0) continue;
         if (!try_lock(lp)) continue;
-        bool ok = ld32(wp) == w && ctr_count(ld64(ctr_of(sb))) == 0;
+        bool ok = ul32(wp) == w && ctr_count(ul64(ctr_of(P, sb))) == 0;
         bool freed = false;
         if (ok) {
           st32(wp, SB_NONE);
-          if (which == 1) a_add32(ha_p.active, ~0u);  // the pair no longer holds a head
-          u32* l = ha_p.sb_lock + sb;
+          if (which == 1) a_add32(P.active, ~0u);  // the pair no longer holds a head
+          u32* l = P.sb_lock + sb;
           lock(l);
-          freed = detach_head(sb);
+          freed = detach_head(P, sb);
           unlock(l);
         }
         unlock(lp);
@@ -281,18 +310,18 @@ constexpr u32 MAX_STEALS = 4;
 
 // With several head sets, free slabs are scarce below the largest of nheads,
 // half the (head set, class) pairs that hold a head, and a quarter of the heap.
-HA_DEV bool free_scarce() {
-  if (ha_p.nheads <= 1) return false;
+HA_DEV bool free_scarce(const Params& P) {
+  if (P.nheads <= 1) return false;
   u32 n = 0;
-  u64* w = set_words(0);
-  for (u32 i = 0; i < ha_p.nsw; ++i) n += (u32)__builtin_popcountll(ld64(w + i));
-  u32 lim = ld32(ha_p.active) / 2;
-  lim = lim > ha_p.nheads ? lim : ha_p.nheads;
-  lim = lim > ha_p.nsbs / 4 ? lim : ha_p.nsbs / 4;
+  u64* w = set_words(P, 0);
+  for (u32 i = 0; i < P.nsw; ++i) n += (u32)__builtin_popcountll(ul64(w + i));
+  u32 lim = ul32(P.active) / 2;
+  lim = lim > P.nheads ? lim : P.nheads;
+  lim = lim > P.nsbs / 4 ? lim : P.nsbs / 4;
   return n < lim;
 }
 
-HA_DEV u32 adopt_head(u32 ihead, u32 size_id);
+HA_DEV u32 adopt_head(const Params& P, u32 ihead, u32 size_id);
 
 // find_sb_for_size (src/slab.cuh:259-372): roomy -> sparse -> free -> busy;
 // for a head needed now, first (after sparse) a head of the class that a pair
@@ -302,99 +331,99 @@ HA_DEV u32 adopt_head(u32 ihead, u32 size_id);
 // that another class holds idle (steal_idle_head, other_idle) and, if none,
 // tries sharing: pairs that share a head put two ticket sequences into one
 // slab and crowd it.
-HA_DEV u32 find_sb_for_size(u32 size_id, u32 chunk_id, u32 ihead, bool now) {
-  const SizeInfo& s = ha_p.si[size_id];
+HA_DEV u32 find_sb_for_size(const Params& P, u32 size_id, u32 chunk_id, u32 ihead, bool now) {
+  const SizeInfo& s = P.si[size_id];
   u32 sb;
   bool tried_share = false, tried_idle = false;
   u32 nsteal = 0;
 again:
-  while ((sb = set_pop(set_roomy(size_id))) != SB_NONE) {
-    Desc* d = ha_p.desc + sb;
-    u32* l = ha_p.sb_lock + sb;
+  while ((sb = set_pop(P, set_roomy(size_id))) != SB_NONE) {
+    Desc* d = P.desc + sb;
+    u32* l = P.sb_lock + sb;
     lock(l);
     bool found = false;
-    if (!ld32(&d->is_head) && ld32(&d->size_id) == size_id) {
-      if (ctr_count(ld64(ctr_of(sb))) <= s.roomy_thr) {
+    if (!ul32(&d->is_head) && ul32(&d->size_id) == size_id) {
+      if (ctr_count(ul64(ctr_of(P, sb))) <= s.roomy_thr) {
         found = true;
         st32(&d->is_head, 1);
-        a_add(ctr_of(sb), CTR_HEAD);
+        a_add(ctr_of(P, sb), CTR_HEAD);
       } else {
-        set_add(set_busy(size_id), sb);
+        set_add(P, set_busy(size_id), sb);
       }
     }
     unlock(l);
     if (found) return sb;
   }
-  while ((sb = set_pop(set_sparse(chunk_id))) != SB_NONE) {
-    Desc* d = ha_p.desc + sb;
-    u32* l = ha_p.sb_lock + sb;
+  while ((sb = set_pop(P, set_sparse(chunk_id))) != SB_NONE) {
+    Desc* d = P.desc + sb;
+    u32* l = P.sb_lock + sb;
     lock(l);
     bool found = false;
-    if (!ld32(&d->is_head) && ld32(&d->chunk_id) == chunk_id) {
-      if (ctr_count(ld64(ctr_of(sb))) <= s.sparse_thr) {
+    if (!ul32(&d->is_head) && ul32(&d->chunk_id) == chunk_id) {
+      if (ctr_count(ul64(ctr_of(P, sb))) <= s.sparse_thr) {
         found = true;
         st32(&d->is_head, 1);
         st32(&d->size_id, size_id);
-        a_add(ctr_of(sb), CTR_HEAD);
+        a_add(ctr_of(P, sb), CTR_HEAD);
       } else {
-        set_add(set_roomy(ld32(&d->size_id)), sb);
+        set_add(P, set_roomy(ul32(&d->size_id)), sb);
       }
     }
     unlock(l);
     if (found) return sb;
   }
   if (now) {
-    const u32 a = adopt_head(ihead, size_id);
+    const u32 a = adopt_head(P, ihead, size_id);
     if (a != SB_NONE) return a;
   }
-  const bool scarce = free_scarce();
+  const bool scarce = free_scarce(P);
   if (scarce && !now) return SB_NONE;
   bool freed_idle = false;
   if (scarce && now && !tried_idle) {
     tried_idle = true;
-    freed_idle = steal_idle_head(ihead, size_id, true);
+    freed_idle = steal_idle_head(P, ihead, size_id, true);
   }
   if (scarce && now && !freed_idle && !tried_share) {
     tried_share = true;
-    u32 shared = share_head(ihead, size_id, chunk_id);
+    u32 shared = share_head(P, ihead, size_id, chunk_id);
     if (shared != SB_NONE) return shared;
   }
-  while ((sb = set_pop(0)) != SB_NONE) {
-    Desc* d = ha_p.desc + sb;
-    u32* l = ha_p.sb_lock + sb;
+  while ((sb = set_pop(P, 0)) != SB_NONE) {
+    Desc* d = P.desc + sb;
+    u32* l = P.sb_lock + sb;
     lock(l);
     bool found = false;
-    if (!ld32(&d->is_head)) {
+    if (!ul32(&d->is_head)) {
       found = true;
       st32(&d->is_head, 1);
       st32(&d->size_id, size_id);
       st32(&d->chunk_id, chunk_id);
       st32(&d->chunk_sz, s.chunk_sz);
-      a_add(ctr_of(sb), CTR_HEAD);
-      a_sub(ctr_of(sb), ctr_chunk_delta(chunk_id));
+      a_add(ctr_of(P, sb), CTR_HEAD);
+      a_sub(ctr_of(P, sb), ctr_chunk_delta(chunk_id));
     }
     unlock(l);
     if (found) return sb;
   }
-  u64* w = set_words(set_busy(size_id));
+  u64* w = set_words(P, set_busy(size_id));
   u32 limit = (s.busy_thr + s.nchunks) / 2;
-  for (u32 i = 0; i < ha_p.nsw; ++i) {
-    u64 word = ld64(w + i);
+  for (u32 i = 0; i < P.nsw; ++i) {
+    u64 word = ul64(w + i);
     while (word) {
       u32 b = (u32)__builtin_ctzll(word);
       u64 m = 1ull << b;
       word &= ~m;
       sb = i * 64 + b;
-      if (ctr_count(ld64(ctr_of(sb))) >= limit) continue;  // a head is swapped out at limit
-      if (!(a_and(w + i, ~m) & m)) continue;
-      Desc* d = ha_p.desc + sb;
-      u32* l = ha_p.sb_lock + sb;
+      if (ctr_count(ul64(ctr_of(P, sb))) >= limit) continue;  // a head is swapped out at limit
+      if (!(rfl64(a_and(w + i, ~m)) & m)) continue;
+      Desc* d = P.desc + sb;
+      u32* l = P.sb_lock + sb;
       lock(l);
       bool found = false;
-      if (!ld32(&d->is_head) && ld32(&d->size_id) == size_id) {
+      if (!ul32(&d->is_head) && ul32(&d->size_id) == size_id) {
         found = true;
         st32(&d->is_head, 1);
-        a_add(ctr_of(sb), CTR_HEAD);
+        a_add(ctr_of(P, sb), CTR_HEAD);
       }
       unlock(l);
       if (found) return sb | HEAD_EXT;
@@ -403,10 +432,10 @@ again:
   if (!now) return SB_NONE;
   if (!tried_share) {
     tried_share = true;
-    u32 shared = share_head(ihead, size_id, chunk_id);
+    u32 shared = share_head(P, ihead, size_id, chunk_id);
     if (shared != SB_NONE) return shared;
   }
-  if (nsteal < MAX_STEALS && steal_idle_head(ihead, size_id)) {
+  if (nsteal < MAX_STEALS && steal_idle_head(P, ihead, size_id)) {
     ++nsteal;
     goto again;
   }
@@ -421,12 +450,12 @@ again:
 // heads of every class seen stay within a third of the heap.
 
 // spread for ncl classes (a power of two, at most nheads, at least 1)
-HA_DEV u32 spread_for(u32 ncl) {
-  const u32 per = ha_p.nsbs / (3u * (ncl ? ncl : 1u));
-  if (per >= ha_p.nheads) return ha_p.nheads;
+HA_DEV u32 spread_for(const Params& P, u32 ncl) {
+  const u32 per = P.nsbs / (3u * (ncl ? ncl : 1u));
+  if (per >= P.nheads) return P.nheads;
   u32 s = 1;
-  while (2 * s <= per && 2 * s <= ha_p.nheads) s *= 2;
-  return s >= ha_p.nheads ? ha_p.nheads : s;
+  while (2 * s <= per && 2 * s <= P.nheads) s *= 2;
+  return s >= P.nheads ? P.nheads : s;
 }
 
 // Size class c holds a head for the first time: count it and shrink the
@@ -436,19 +465,19 @@ HA_DEV u32 spread_for(u32 ncl) {
 // (adopt_head), while their empty heads and cached heads go to whichever
 // search needs a slab (steal_idle_head).  No head is detached under waves
 // that may still be reserving in it.
-HA_DEV void note_class(u32 c) {
-  if (ha_p.fixed_sets) return;
+HA_DEV void note_class(const Params& P, u32 c) {
+  if (P.fixed_sets) return;
   const u32 bit = 1u << c;
-  if (ld32(ha_p.class_seen) & bit) return;
-  const u32 old = __hip_atomic_fetch_or(ha_p.class_seen, bit, __ATOMIC_RELAXED, HA_SCOPE);
+  if (ul32(P.class_seen) & bit) return;
+  const u32 old = rfl(__hip_atomic_fetch_or(P.class_seen, bit, __ATOMIC_RELAXED, HA_SCOPE));
   if (old & bit) return;
-  const u32 want = spread_for((u32)__builtin_popcount(old | bit));
-  u32 cur = ld32(ha_p.spread);
+  const u32 want = spread_for(P, (u32)__builtin_popcount(old | bit));
+  u32 cur = ul32(P.spread);
   while (want < cur) {
     u32 e = cur;
-    if (__hip_atomic_compare_exchange_strong(ha_p.spread, &e, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                             HA_SCOPE))
-      break;
+    (void)__hip_atomic_compare_exchange_strong(P.spread, &e, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED, HA_SCOPE);
+    e = rfl(e);  // the value found
+    if (e == cur) break;
     cur = e;
   }
 }
@@ -457,21 +486,21 @@ HA_DEV void note_class(u32 c) {
 // the word moves to the caller's pair, the slab stays a head with the same
 // reference, so waves still reserving in it stay consistent.  Caller holds
 // the head lock of (ihead, size_id); the other pair's lock is only tried.
-HA_DEV u32 adopt_head(u32 ihead, u32 size_id) {
-  if (ha_p.fixed_sets) return SB_NONE;
-  const SizeInfo& s = ha_p.si[size_id];
-  for (u32 ih = ld32(ha_p.spread); ih < ha_p.nheads; ++ih) {
+HA_DEV u32 adopt_head(const Params& P, u32 ihead, u32 size_id) {
+  if (P.fixed_sets) return SB_NONE;
+  const SizeInfo& s = P.si[size_id];
+  for (u32 ih = ul32(P.spread); ih < P.nheads; ++ih) {
     if (ih == ihead) continue;
-    u32* hp = hot(ha_p.head, ih, size_id);
-    u32 w = ld32(hp);
-    if (w == SB_NONE || ctr_count(ld64(ctr_of(w & ~HEAD_EXT))) >= head_limit(w, s)) continue;
-    u32* lp = hot(ha_p.head_lock, ih, size_id);
+    u32* hp = hot(P.head, ih, size_id);
+    u32 w = ul32(hp);
+    if (w == SB_NONE || ctr_count(ul64(ctr_of(P, w & ~HEAD_EXT))) >= head_limit(w, s)) continue;
+    u32* lp = hot(P.head_lock, ih, size_id);
     if (!try_lock(lp)) continue;
-    w = ld32(hp);
+    w = ul32(hp);
     const bool ok = w != SB_NONE;
     if (ok) {
       st32(hp, SB_NONE);
-      a_add32(ha_p.active, ~0u);  // that pair no longer holds a head
+      a_add32(P.active, ~0u);  // that pair no longer holds a head
     }
     unlock(lp);
     if (ok) return w;
@@ -494,44 +523,46 @@ HA_DEV u32 adopt_head(u32 ihead, u32 size_id) {
 // of the same head before any slab has become free keeps it without
 // searching again.
 HA_DEV u32 new_sb_for_size(u32 size_id, u32 ihead, u32 seen, bool force = false) {
-  const SizeInfo& s = ha_p.si[size_id];
-  if (!ha_p.fixed_sets) {
+  size_id = rfl(size_id), ihead = rfl(ihead), seen = rfl(seen);
+  const Params& P = params();
+  const SizeInfo& s = P.si[size_id];
+  if (!P.fixed_sets) {
     // a wave with a stale spread names a pair outside the spread: serve it
     // from the pair its set folds onto.  `seen` stays the head the caller
     // last used: when that is the folded pair's head, it is replaced as for
     // any caller of that pair
-    const u32 sp = ld32(ha_p.spread);
-    if (ihead >= sp) ihead = fold_set(ihead, sp);
+    const u32 sp = ul32(P.spread);
+    if (ihead >= sp) ihead = fold_set(P, ihead, sp);
   }
-  u32* hp = hot(ha_p.head, ihead, size_id);
-  u32* lp = hot(ha_p.head_lock, ihead, size_id);
-  u32* cp = hot(ha_p.cached, ihead, size_id);
-  u32* ep = hot(ha_p.search_ep, ihead, size_id);
-  u32* fp = hot(ha_p.forced, ihead, size_id);  // [0] head word, [1] free epoch
+  u32* hp = hot(P.head, ihead, size_id);
+  u32* lp = hot(P.head_lock, ihead, size_id);
+  u32* cp = hot(P.cached, ihead, size_id);
+  u32* ep = hot(P.search_ep, ihead, size_id);
+  u32* fp = hot(P.forced, ihead, size_id);  // [0] head word, [1] free epoch
   for (;;) {
-    u32 cur = ld32(hp);
+    u32 cur = ul32(hp);
     if (cur != seen && cur != SB_NONE) return cur;
-    const u32 e0 = ld32(ep);
+    const u32 e0 = ul32(ep);
     if (try_lock(lp)) {
-      cur = ld32(hp);
+      cur = ul32(hp);
       u32 nh;
       // below: a forced replacement of a head that still has room
-      const bool below = cur != SB_NONE && ctr_count(ld64(ctr_of(cur & ~HEAD_EXT))) < head_limit(cur, s);
-      const u32 fe = ld32(ha_p.free_ep);
-      if (below && ld32(fp) == cur && ld32(fp + 1) == fe) {
+      const bool below = cur != SB_NONE && ctr_count(ul64(ctr_of(P, cur & ~HEAD_EXT))) < head_limit(cur, s);
+      const u32 fe = ul32(P.free_ep);
+      if (below && ul32(fp) == cur && ul32(fp + 1) == fe) {
         nh = cur;  // this head's forced search failed, and no slab became free since
       } else if (cur == SB_NONE || !below || (force && cur == seen)) {
-        nh = ld32(cp);
+        nh = ul32(cp);
         st32(cp, SB_NONE);
         if (nh == SB_NONE) {
           // one head search per class at a time: a pair that follows sees the
           // head the one before it took and can share it instead of taking
           // another slab
-          u32* cl = ha_p.class_lock + size_id * HOT_STRIDE;
-          if (ha_p.nheads > 1) lock(cl);
-          nh = find_sb_for_size(size_id, s.chunk_id, ihead, true);
-          if (ha_p.nheads > 1) unlock(cl);
-          st32(ep, (((ld32(ep) >> 1) + 1) << 1) | (nh == SB_NONE && !below ? 1u : 0u));
+          u32* cl = P.class_lock + size_id * HOT_STRIDE;
+          if (P.nheads > 1) lock(cl);
+          nh = find_sb_for_size(P, size_id, s.chunk_id, ihead, true);
+          if (P.nheads > 1) unlock(cl);
+          st32(ep, (((ul32(ep) >> 1) + 1) << 1) | (nh == SB_NONE && !below ? 1u : 0u));
         }
         if (nh == SB_NONE && below) {
           nh = cur;  // no other slab: keep the head, which still has room
@@ -541,17 +572,17 @@ HA_DEV u32 new_sb_for_size(u32 size_id, u32 ihead, u32 seen, bool force = false)
           __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
           st32(hp, nh);
           if (cur == SB_NONE) {
-            a_add32(ha_p.active, 1u);
-            note_class(size_id);
+            a_add32(P.active, 1u);
+            note_class(P, size_id);
           }
           if (cur != SB_NONE) {
             u32 csb = cur & ~HEAD_EXT;
-            u32* l = ha_p.sb_lock + csb;
+            u32* l = P.sb_lock + csb;
             lock(l);
-            detach_head(csb);
+            detach_head(P, csb);
             unlock(l);
           }
-          st32(cp, find_sb_for_size(size_id, s.chunk_id, ihead, false));
+          st32(cp, find_sb_for_size(P, size_id, s.chunk_id, ihead, false));
         }
       } else {
         nh = cur;
@@ -559,10 +590,10 @@ HA_DEV u32 new_sb_for_size(u32 size_id, u32 ihead, u32 seen, bool force = false)
       unlock(lp);
       return nh;
     }
-    while (ld32(hp) == cur && ld32(lp) != 0) __builtin_amdgcn_s_sleep(2);
+    while (ul32(hp) == cur && ul32(lp) != 0) __builtin_amdgcn_s_sleep(2);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    const u32 e1 = ld32(ep);
-    if (e1 != e0 && (e1 & 1u) && ld32(hp) == cur) return SB_NONE;
+    const u32 e1 = ul32(ep);
+    if (e1 != e0 && (e1 & 1u) && ul32(hp) == cur) return SB_NONE;
   }
 }
 
@@ -586,7 +617,7 @@ HA_DEV u32 mod_chunks(const SizeInfo& s, u64 x) {
 // nibbles, and leaves each reserved lane's chunk in my_ich.  itry advances for
 // the whole group; off0 is the probe offset of the first attempt (a run that
 // resumes after a first attempt made elsewhere starts at itry 1).
-HA_DEV u64 probe_run(const SizeInfo& s, u32 hsb, u32 limit, u32 old, u64 P, u32 me, u32& itry, u32& my_ich,
+HA_DEV u64 probe_run(const Params& P_, const SizeInfo& s, u32 hsb, u32 limit, u32 old, u64 P, u32 me, u32& itry, u32& my_ich,
                      u64 off0 = 0, bool* spent = nullptr) {
   const u32 k = s.ncib, nchunks = s.nchunks, nwb = nchunks >> 6, nwn = nchunks >> 4;
   const u32 slot0 = old & (RUN - 1), split = RUN - slot0;
@@ -595,8 +626,8 @@ HA_DEV u64 probe_run(const SizeInfo& s, u32 hsb, u32 limit, u32 old, u64 P, u32 
   const bool inA = me < split;
   const u64 amask = split >= 64 ? ~0ull : ((1ull << split) - 1);
   const u64 myseg = inA ? amask : ~amask;
-  u64* bw = ha_p.bits + (u64)hsb * ha_p.bit_words;
-  u64* nw = ha_p.nibs + (u64)hsb * ha_p.nib_words;
+  u64* bw = bits_of(P_, hsb);
+  u64* nw = nibs_of(P_, hsb);
   u64 reserved = 0;
   u64 off = off0;
   for (;;) {
@@ -637,7 +668,7 @@ HA_DEV u64 probe_run(const SizeInfo& s, u32 hsb, u32 limit, u32 old, u64 P, u32 
     P = F;
     if (!P) break;
     if (itry % CHECK_NTRIES == CHECK_NTRIES - 1) {
-      if (ctr_count(ld64(ctr_of(hsb))) >= limit) break;
+      if (ctr_count(ld64(ctr_of(P_, hsb))) >= limit) break;
     }
     const u32 step = mod_by((itry + 1) * STEP_FREQ * k, s.hash_step, s.hash_step_m);
     off = (u64)(itry + 1) * step;
@@ -651,28 +682,31 @@ HA_DEV u64 probe_run(const SizeInfo& s, u32 hsb, u32 limit, u32 old, u64 P, u32 
 
 // gives back one reserved block of this lane: nibble first, then the bits
 HA_DEV void release_block(u32 hsb, u32 ich, u32 k) {
-  a_and(ha_p.nibs + (u64)hsb * ha_p.nib_words + ich / 16, ~(0xFull << (4 * (ich % 16))));
+  const Params& P = params();
+  a_and(nibs_of(P, hsb) + ich / 16, ~(0xFull << (4 * (ich % 16))));
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-  a_and(ha_p.bits + (u64)hsb * ha_p.bit_words + ich / 64, ~(((1ull << k) - 1) << (ich % 64)));
+  a_and(bits_of(P, hsb) + ich / 64, ~(((1ull << k) - 1) << (ich % 64)));
 }
 
 // One size class of one wave (hamalloc_small, src/halloc.cu:125-182).  The
 // active lanes are exactly the bitmap g; sid, g and ihead are wave-uniform.
 HA_DEV void* malloc_group(u32 sid, u64 g, u32 ihead, u32 me) {
-  const SizeInfo& s = ha_p.si[sid];
-  const u32 k = s.ncib;
   const u32 lead = (u32)__builtin_ctzll(g);
   const u32 last = 63u - (u32)__builtin_clzll(g);
-  u32 hword = rfl(ld32(hot(ha_p.head, ihead, sid)));
+  const Params& P0 = params();
+  u32 hword = rfl(ld32(hot(P0.head, ihead, sid)));
   // tickets (size_ctr_inc, src/halloc.cu:71-98): one atomic per group
   u32 old = 0;
-  if (me == lead) old = a_add32(hot(ha_p.ticket, ihead, sid), last + 1);
+  if (me == lead) old = a_add32(hot(P0.ticket, ihead, sid), last + 1);
   old = rdl(old, lead);
   u32 itry = 0;
   u64 want = g;
   void* p = nullptr;
   u32 my_ich = 0;
   while (want) {
+    const Params& P = params();  // read again after a head replacement rather than held over it
+    const SizeInfo& s = P.si[sid];
+    const u32 k = s.ncib;
     bool need = false, spent = false, crowded = false;
     const u32 hsb = hword == SB_NONE ? SB_NONE : (hword & ~HEAD_EXT);
     const u32 limit = head_limit(hword, s);
@@ -680,7 +714,7 @@ HA_DEV void* malloc_group(u32 sid, u64 g, u32 ihead, u32 me) {
       need = true;
     } else {
       const u32 itry0 = itry;
-      const u64 reserved = probe_run(s, hsb, limit, old, want, me, itry, my_ich, 0, &spent);
+      const u64 reserved = probe_run(P, s, hsb, limit, old, want, me, itry, my_ich, 0, &spent);
       if (reserved != want) need = true;
       // a probe sequence this long says the head is crowded: the group's last
       // lanes wait for the luckiest of log(64) / log(1 / fill) rounds, so the
@@ -690,21 +724,21 @@ HA_DEV void* malloc_group(u32 sid, u64 g, u32 ihead, u32 me) {
         // sb_ctr_inc (src/slab.cuh:122-155): one atomic for the group
         const u32 change = k * (u32)__builtin_popcountll(reserved);
         u64 oldc = 0;
-        if (me == lead) oldc = a_add(ctr_of(hsb), (u64)change << CTR_COUNT_SH);
+        if (me == lead) oldc = a_add(ctr_of(P, hsb), (u64)change << CTR_COUNT_SH);
         oldc = rdl64(oldc, lead);
         const bool mine = (reserved >> me) & 1;
         if (ctr_chunk(oldc) != s.chunk_id) {
           // the slab was freed under us: give the chunks back
           if (mine) release_block(hsb, my_ich, k);
           if (me == lead) {
-            u64 o = a_sub(ctr_of(hsb), (u64)change << CTR_COUNT_SH);
+            u64 o = a_sub(ctr_of(P, hsb), (u64)change << CTR_COUNT_SH);
             ctr_transitions(hsb, o, change);
           }
           need = true;
         } else {
           const u32 oc = ctr_count(oldc);
           if (oc < limit && oc + change >= limit) need = true;
-          if (mine) p = ha_p.arena + (u64)hsb * ha_p.sb_sz + chunk_mul(my_ich, s.chunk_sz);
+          if (mine) p = slab_of(P, hsb) + chunk_mul(my_ich, s.chunk_sz);
           want &= ~reserved;
         }
       }
@@ -749,7 +783,8 @@ HA_DEV BatchProbe batch_probe(const SizeInfo& s, u32 old, u32 me, u64 P) {
 // calls would be), every round probed in the current head, ONE counter atomic
 // for all reserved chunks; unserved lanes and rollbacks go through plain rounds.
 HA_DEV void malloc_batch_group(u32 sid, u64 g, u32 ihead, u32 me, u32 cnt, void** out) {
-  const SizeInfo& s = ha_p.si[sid];
+  const Params& P_ = params();
+  const SizeInfo& s = P_.si[sid];
   const u32 k = s.ncib;
   const u32 lead = (u32)__builtin_ctzll(g);
   const u32 L = 64u - (u32)__builtin_clzll(g);
@@ -759,8 +794,8 @@ HA_DEV void malloc_batch_group(u32 sid, u64 g, u32 ihead, u32 me, u32 cnt, void*
   // the ticket and the head load go out together: no head search touches a
   // ticket, so taking it before a missing head is replaced changes nothing
   u32 base = 0;
-  if (me == lead) base = a_add32(hot(ha_p.ticket, ihead, sid), R * L);
-  u32 hword = rfl(ld32(hot(ha_p.head, ihead, sid)));
+  if (me == lead) base = a_add32(hot(P_.ticket, ihead, sid), R * L);
+  u32 hword = rfl(ld32(hot(P_.head, ihead, sid)));
   base = rdl(base, lead);
   if (hword == SB_NONE) {  // no head yet: get one first
     u32 nh = 0;
@@ -775,10 +810,10 @@ HA_DEV void malloc_batch_group(u32 sid, u64 g, u32 ihead, u32 me, u32 cnt, void*
     need = true;
   } else {
     u32 total = 0;
-    char* sbase = ha_p.arena + (u64)hsb * ha_p.sb_sz;
+    char* sbase = slab_of(P_, hsb);
     const u32 nchunks = s.nchunks, nwn = nchunks >> 4;
-    u64* bw = ha_p.bits + (u64)hsb * ha_p.bit_words;
-    u64* nw = ha_p.nibs + (u64)hsb * ha_p.nib_words;
+    u64* bw = bits_of(P_, hsb);
+    u64* nw = nibs_of(P_, hsb);
     // the first probe of every round is issued before any result is awaited;
     // then, round by round, the lanes that failed give their new bits back and
     // go on from the second probe.  ow is indexed by the wave-uniform round, so
@@ -823,7 +858,7 @@ HA_DEV void malloc_batch_group(u32 sid, u64 g, u32 ihead, u32 me, u32 cnt, void*
         // resume at the second probe (itry 1) for the lanes left over
         u32 itry = 1, my_ich = 0;
         const u64 off1 = (u64)mod_by(STEP_FREQ * k, s.hash_step, s.hash_step_m);
-        const u64 S2 = probe_run(s, hsb, limit, base + j * L, F, me, itry, my_ich, off1);
+        const u64 S2 = probe_run(P_, s, hsb, limit, base + j * L, F, me, itry, my_ich, off1);
         if ((S2 >> me) & 1) out[j] = sbase + chunk_mul(my_ich, s.chunk_sz);
         Sall |= S2;
       }
@@ -833,7 +868,7 @@ HA_DEV void malloc_batch_group(u32 sid, u64 g, u32 ihead, u32 me, u32 cnt, void*
     if (total) {
       const u32 change = k * total;
       u64 oldc = 0;
-      if (me == lead) oldc = a_add(ctr_of(hsb), (u64)change << CTR_COUNT_SH);
+      if (me == lead) oldc = a_add(ctr_of(P_, hsb), (u64)change << CTR_COUNT_SH);
       oldc = rdl64(oldc, lead);
       if (ctr_chunk(oldc) != s.chunk_id) {
         for (u32 j = 0; j < cnt; ++j) {
@@ -841,7 +876,7 @@ HA_DEV void malloc_batch_group(u32 sid, u64 g, u32 ihead, u32 me, u32 cnt, void*
           out[j] = nullptr;
         }
         if (me == lead) {
-          u64 o = a_sub(ctr_of(hsb), (u64)change << CTR_COUNT_SH);
+          u64 o = a_sub(ctr_of(P_, hsb), (u64)change << CTR_COUNT_SH);
           ctr_transitions(hsb, o, change);
         }
         need = true;
@@ -888,18 +923,22 @@ HA_DEV void free_rounds(const u64* off, const bool* act) {
   // the blocks, or a later eviction of this XCD's dirty lines would overwrite
   // the new owner's data: one agent-scope release per wave call.  The default
   // uncached arena needs none.
-  if (ha_p.cached_arena) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+  const Params& P = params();
+  if (P.cached_arena) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
   const u32 me = lane_id();
   u32 sb[NR], cs[NR], sid[NR], cid[NR];
 #pragma unroll
   for (int j = 0; j < NR; ++j) {
-    sb[j] = act[j] ? (u32)(off[j] >> ha_p.sb_sz_sh) : 0u;
+    sb[j] = act[j] ? (u32)(off[j] >> P.sb_sz_sh) : 0u;
     cs[j] = sid[j] = cid[j] = 0;
     if (act[j]) {
-      Desc* d = ha_p.desc + sb[j];
-      cs[j] = ld32(&d->chunk_sz);
-      sid[j] = ld32(&d->size_id);
-      cid[j] = ld32(&d->chunk_id);
+      Desc* d = P.desc + sb[j];
+      // size id and chunk id in one load; the chunk size follows from the id
+      // (16, 24, 256 or 384 B: 2 or 3 units of 8 or 128, kept as div3 << 16 | shift)
+      const u64 w = ld64((u64*)d);
+      sid[j] = (u32)w;
+      cid[j] = (u32)(w >> 32);
+      cs[j] = cid[j] == SZ_NONE ? 0u : ((cid[j] & 1) ? 3u << 16 | 3u : 1u << 16 | 4u) + (cid[j] >> 1) * 4u;
     }
   }
   // nibbles: read back the block lengths and clear them
@@ -910,7 +949,7 @@ HA_DEV void free_rounds(const u64* off, const bool* act) {
 #pragma unroll
   for (int j = 0; j < NR; ++j) {
     const bool valid = act[j] && cs[j] != 0;
-    ich[j] = valid ? chunk_div((u32)(off[j] & (ha_p.sb_sz - 1)), cs[j]) : 0u;
+    ich[j] = valid ? chunk_div((u32)(off[j] & (P.sb_sz - 1)), cs[j]) : 0u;
     A[j] = ballot(valid);
     nch[j] = 0;
     k[j] = st[j] = 0;
@@ -925,7 +964,7 @@ HA_DEV void free_rounds(const u64* off, const bool* act) {
       if (ballot(valid && sb[j] == sb0) == A[j]) {
         const u32 sid0 = rdl(sid[j], l0);
         if (sid0 < NSIZES) {
-          k[j] = ha_p.si[sid0].ncib;
+          k[j] = P.si[sid0].ncib;
           const u32 sa = rdl(ich[j], l0) - l0 * k[j];
           const bool ina = valid && ich[j] == sa + me * k[j];
           const u64 Am = ballot(ina);
@@ -946,7 +985,7 @@ HA_DEV void free_rounds(const u64* off, const bool* act) {
         }
       }
     }
-    u64* nw = ha_p.nibs + (u64)sb[j] * ha_p.nib_words;
+    u64* nw = nibs_of(P, sb[j]);
     if (fast[j]) {
       u32 wn;
       u64 un;
@@ -960,7 +999,7 @@ HA_DEV void free_rounds(const u64* off, const bool* act) {
 #pragma unroll
   for (int j = 0; j < NR; ++j) {
     const bool valid = act[j] && cs[j] != 0;
-    u64* bw = ha_p.bits + (u64)sb[j] * ha_p.bit_words;
+    u64* bw = bits_of(P, sb[j]);
     if (fast[j]) {
       const u64 oldn = shfl64(o[j], inn[j] & 63);
       nch[j] = valid ? (u32)((oldn >> (4 * (ich[j] & 15))) & 0xF) : 0u;
@@ -1008,15 +1047,15 @@ HA_DEV void free_rounds(const u64* off, const bool* act) {
       rem &= ~G;
     }
     oldc[j] = 0;
-    if (leader) oldc[j] = a_sub(ctr_of(sb[j]), (u64)my_change << CTR_COUNT_SH);
+    if (leader) oldc[j] = a_sub(ctr_of(P, sb[j]), (u64)my_change << CTR_COUNT_SH);
     change[j] = my_change;
     lead[j] = leader;
   }
 #pragma unroll
   for (int j = 0; j < NR; ++j) {
     const bool tr = lead[j] && !ctr_is_head(oldc[j]) && sid[j] < NSIZES && cid[j] != SZ_NONE &&
-                    sb_class(ctr_count(oldc[j]), ha_p.si[sid[j]]) !=
-                        sb_class(ctr_count(oldc[j]) - change[j], ha_p.si[sid[j]]);
+                    sb_class(ctr_count(oldc[j]), P.si[sid[j]]) !=
+                        sb_class(ctr_count(oldc[j]) - change[j], P.si[sid[j]]);
     u64 T = ballot(tr);
     while (T) {
       const u32 l = (u32)__builtin_ctzll(T);
@@ -1068,6 +1107,7 @@ HA_DEV u32 next_lane(u64& walk) {
 }
 
 HA_DEV void free_runs(u32 F, RunRounds r) {
+  const Params& P = params();
   const u32 me = lane_id();
   const u64 lanes = ballot(true);
   const u32 jme = (u32)__builtin_popcountll(lanes & ((1ull << me) - 1));  // the round this lane holds
@@ -1085,7 +1125,7 @@ HA_DEV void free_runs(u32 F, RunRounds r) {
       u32 wn, inn;
       u64 un;
       run_word_nibs(x.ina ? x.Am : x.Bm, me, x.st, x.k, 0xFull, wn, un, inn);
-      if (x.act && inn == me) v = a_and(ha_p.nibs + (u64)x.sb * ha_p.nib_words + wn, ~un);
+      if (x.act && inn == me) v = a_and(nibs_of(P, x.sb) + wn, ~un);
     }
     o[j] = v;
   }
@@ -1104,7 +1144,7 @@ HA_DEV void free_runs(u32 F, RunRounds r) {
     const u64 oj = o[j];
     // each issuer checks its own word: every block it cleared was k chunks
     const bool bad = x.act && inn == me && (oj & un) != (un / 0xFull) * x.k;
-    u64* bw = ha_p.bits + (u64)x.sb * ha_p.bit_words;
+    u64* bw = bits_of(P, x.sb);
     u32 change;
     if (!ballot(bad)) {
       u32 wb, ib;
@@ -1146,11 +1186,11 @@ HA_DEV void free_runs(u32 F, RunRounds r) {
     rem &= ~G;
   }
   u64 told = 0;
-  if (inF && me == ldr) told = a_sub(ctr_of(rsb), (u64)tot << CTR_COUNT_SH);
+  if (inF && me == ldr) told = a_sub(ctr_of(P, rsb), (u64)tot << CTR_COUNT_SH);
   const u64 oldc = shfl64(told, ldr) - ((u64)pre << CTR_COUNT_SH);
   const bool tr = inF && !ctr_is_head(oldc) && rsid < NSIZES && rcid != SZ_NONE &&
-                  sb_class(ctr_count(oldc), ha_p.si[rsid < NSIZES ? rsid : 0]) !=
-                      sb_class(ctr_count(oldc) - rch, ha_p.si[rsid < NSIZES ? rsid : 0]);
+                  sb_class(ctr_count(oldc), P.si[rsid < NSIZES ? rsid : 0]) !=
+                      sb_class(ctr_count(oldc) - rch, P.si[rsid < NSIZES ? rsid : 0]);
   for (u64 T = ballot(tr); T; T &= T - 1) {
     const u32 l = (u32)__builtin_ctzll(T);
     if (me == l) ctr_transitions(rsb, oldc, rch);
@@ -1197,11 +1237,12 @@ constexpr u64 UNIT_NONE = ~0ull;
 // large_start(ticket + rank) on, each word claimed by a compare-and-swap from
 // zero.  Returns this lane's unit (UNIT_NONE: nothing free was found).
 HA_DEV u64 large_group(u32 c, u64 g, u32 me) {
+  const Params& P = params();
   const u32 lead = (u32)__builtin_ctzll(g);
-  const u32 nw = ha_p.lwords;
-  u64* lb = ha_p.lbits;
+  const u32 nw = P.lwords;
+  u64* lb = P.lbits;
   u32 old = 0;
-  if (me == lead) old = a_add32(ha_p.lticket + c * HOT_STRIDE, (u32)__builtin_popcountll(g));
+  if (me == lead) old = a_add32(P.lticket + c * HOT_STRIDE, (u32)__builtin_popcountll(g));
   old = rdl(old, lead);
   u64 unit = UNIT_NONE;
   if (c <= 6) {
@@ -1258,16 +1299,17 @@ HA_DEV u64 large_group(u32 c, u64 g, u32 me) {
       }
     }
   }
-  if (unit != UNIT_NONE) st32(ha_p.lstart + unit, c + 1);
+  if (unit != UNIT_NONE) st32(P.lstart + unit, c + 1);
   return unit;
 }
 
 // hamalloc for the active lanes whose requests exceed MAX_BLOCK_SZ: one
 // class group at a time, groups ordered by their lowest lane
 HA_DEV void* large_alloc(u64 nbytes) {
+  const Params& P = params();
   const u32 me = lane_id();
   const u32 c = large_class(nbytes);
-  const bool fits = c < ha_p.lnclasses;
+  const bool fits = c < P.lnclasses;
   void* res = nullptr;
   u64 rem = ballot(fits);
   while (rem) {
@@ -1276,7 +1318,7 @@ HA_DEV void* large_alloc(u64 nbytes) {
     const u64 g = ballot(fits && c == gc) & rem;
     if ((g >> me) & 1) {
       const u64 u = large_group(gc, g, me);
-      if (u != UNIT_NONE) res = ha_p.large + (u << LARGE_UNIT_SH);
+      if (u != UNIT_NONE) res = P.large + (u << LARGE_UNIT_SH);
     }
     rem &= ~g;
   }
@@ -1284,18 +1326,19 @@ HA_DEV void* large_alloc(u64 nbytes) {
 }
 
 HA_DEV void large_free(u64 off) {
+  const Params& P = params();
   if (off & ((1ull << LARGE_UNIT_SH) - 1)) return;  // not a unit start: not a block
   const u64 unit = off >> LARGE_UNIT_SH;
-  const u32 s = a_xchg32(ha_p.lstart + unit, 0u);
+  const u32 s = a_xchg32(P.lstart + unit, 0u);
   if (s == 0) return;  // freed already, inside a block, or never handed out
   // with a cached arena the caller's stores to the block reach memory before
   // its units can be handed out again (see free_rounds)
-  if (ha_p.cached_arena) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+  if (P.cached_arena) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
   const u32 c = s - 1;
   if (c <= 6) {
-    a_and(ha_p.lbits + unit / 64, ~(low_mask(1u << c) << (unit % 64)));
+    a_and(P.lbits + unit / 64, ~(low_mask(1u << c) << (unit % 64)));
   } else {
-    for (u64 j = 0; j < (1ull << (c - 6)); ++j) a_and(ha_p.lbits + unit / 64 + j, 0ull);
+    for (u64 j = 0; j < (1ull << (c - 6)); ++j) a_and(P.lbits + unit / 64 + j, 0ull);
   }
 }
 
@@ -1319,7 +1362,7 @@ HA_API void* hamalloc(size_t nbytes) {
   // requests above 3072 B go to the large-block region (src/halloc.cu:185-195
   // sends them to the CUDA device heap)
   if (nbytes > ha::MAX_BLOCK_SZ) return ha::large_alloc(nbytes);
-  return ha::malloc_small((ha::u32)nbytes, ha::rfl(ha::fold_set(ha::head_set(), ha::spread_cached())));
+  return ha::malloc_small((ha::u32)nbytes, ha::wave_set());
 }
 
 // Batched allocation: lane l gets cnt (<= HA_MAX_BATCH) blocks of nbytes into
@@ -1350,7 +1393,7 @@ HA_DEV int malloc_batch_on(size_t nbytes, int cnt, void** out, u32 ihead) {
 }  // namespace ha
 
 HA_API int hamalloc_batch(size_t nbytes, int cnt, void** out) {
-  return ha::malloc_batch_on(nbytes, cnt, out, ha::rfl(ha::fold_set(ha::head_set(), ha::spread_cached())));
+  return ha::malloc_batch_on(nbytes, cnt, out, ha::wave_set());
 }
 
 // Batched free: lane l frees ptrs[0..cnt) (NULL entries are skipped); round
@@ -1361,16 +1404,17 @@ HA_API int hamalloc_batch(size_t nbytes, int cnt, void** out) {
 HA_API void hafree_batch(void* const* ptrs, int cnt) {
   using namespace ha;
   if (cnt <= 0) return;
+  const Params& P = params();
   const u32 c = cnt > (int)MAXB ? MAXB : (u32)cnt;
   u32 R = 0;  // the wave's largest count
   for (u32 j = 0; j < MAXB; ++j)
     if (ballot(c > j)) R = j + 1;
   for (u32 j = 0; j < c; ++j) {
     void* p = ptrs[j];
-    if (p && (u64)((char*)p - ha_p.arena) >= ha_p.arena_bytes) hafree(p);
+    if (p && (u64)((char*)p - P.arena) >= P.arena_bytes) hafree(p);
   }
   // see free_rounds: one release per call for a cached arena
-  if (ha_p.cached_arena) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+  if (P.cached_arena) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
   const u32 me = lane_id();
   // every round's slab, where all its blocks lie in one (the j-th active lane
   // holds round j's; with fewer active lanes than rounds, every round goes
@@ -1387,10 +1431,10 @@ HA_API void hafree_batch(void* const* ptrs, int cnt) {
     if (j >= R) continue;
     const u32 l = held ? next_lane(walk) : 0u;
     void* p = j < c ? ptrs[j] : nullptr;
-    const u64 off = (u64)((char*)p - ha_p.arena);
-    const bool act = p && off < ha_p.arena_bytes;
-    const u32 sb = act ? (u32)(off >> ha_p.sb_sz_sh) : 0u;
-    ino[j] = (u32)(off & (ha_p.sb_sz - 1));
+    const u64 off = (u64)((char*)p - P.arena);
+    const bool act = p && off < P.arena_bytes;
+    const u32 sb = act ? (u32)(off >> P.sb_sz_sh) : 0u;
+    ino[j] = (u32)(off & (P.sb_sz - 1));
     actm |= (u32)act << j;
     const u64 A = ballot(act);
     if (!A || !held) continue;
@@ -1403,7 +1447,7 @@ HA_API void hafree_batch(void* const* ptrs, int cnt) {
   // their descriptors: one load per round
   u32 rcs = 0, rsid = SZ_NONE, rcid = SZ_NONE;
   if (jme < MAXB && ((single >> jme) & 1)) {
-    Desc* d = ha_p.desc + rsb;
+    Desc* d = P.desc + rsb;
     rcs = ld32(&d->chunk_sz);
     rsid = ld32(&d->size_id);
     rcid = ld32(&d->chunk_id);
@@ -1420,7 +1464,7 @@ HA_API void hafree_batch(void* const* ptrs, int cnt) {
     if (cs == 0 || sid >= NSIZES) continue;
     const bool act = (actm >> j) & 1;
     const u32 ich = act ? chunk_div(ino[j], cs) : 0u;
-    const u32 k = ha_p.si[sid].ncib;
+    const u32 k = P.si[sid].ncib;
     const u64 A = ballot(act);
     const u32 l0 = (u32)__builtin_ctzll(A);
     const u32 sa = rdl(ich, l0) - l0 * k;
@@ -1453,7 +1497,7 @@ HA_API void hafree_batch(void* const* ptrs, int cnt) {
     F = 0;
     if (j < R && ballot((actm >> j) & 1)) {
       const bool act = (actm >> j) & 1;
-      u64 off = act ? (u64)((char*)ptrs[j] - ha_p.arena) : 0ull;
+      u64 off = act ? (u64)((char*)ptrs[j] - P.arena) : 0ull;
       free_rounds<1>(&off, &act);
     }
   }
@@ -1464,8 +1508,9 @@ HA_API void hafree_batch(void* const* ptrs, int cnt) {
 // the replay harness uses them to pin behaviour across head sets
 namespace ha {
 HA_DEV u32 fold_coherent(unsigned full) {
-  const u32 f = full % ha_p.nheads;
-  return ha_p.fixed_sets ? f : fold_set(f, ld32(ha_p.spread));
+  const Params& P = params();
+  const u32 f = full % P.nheads;
+  return P.fixed_sets ? f : fold_set(P, f, ld32(P.spread));
 }
 }  // namespace ha
 __device__ void* ha_malloc_on_head(size_t nbytes, unsigned full) {
@@ -1476,14 +1521,15 @@ __device__ int ha_malloc_batch_on_head(size_t nbytes, int cnt, void** out, unsig
   return ha::malloc_batch_on(nbytes, cnt, out, ha::rfl(ha::fold_coherent(full)));
 }
 // the full-spread head set of the calling wave (what hamalloc folds)
-__device__ unsigned ha_head_set_full() { return ha::rfl(ha::head_set()); }
+__device__ unsigned ha_head_set_full() { return ha::rfl(ha::head_set(ha::params())); }
 
 HA_API void hafree(void* p) {
   if (!p) return;  // src/halloc.cu:240
-  const ha::u64 off = (ha::u64)((char*)p - ha::ha_p.arena);
-  const ha::u64 loff = (ha::u64)((char*)p - ha::ha_p.large);
-  if (off < ha::ha_p.arena_bytes) ha::free_small(off);
-  else if (loff < ha::ha_p.large_bytes) ha::large_free(loff);
+  const ha::Params& P = ha::params();
+  const ha::u64 off = (ha::u64)((char*)p - P.arena);
+  const ha::u64 loff = off - P.arena_bytes;  // the large region follows the slabs
+  if (off < P.arena_bytes) ha::free_small(off);
+  else if (loff < P.large_bytes) ha::large_free(loff);
   else free(p);  // not from this heap: the device heap's (src/halloc.cu:244-246)
 }
 
@@ -1793,7 +1839,7 @@ __global__ void __launch_bounds__(STAT_BS) free_mem_part_k(u64* buf) {
   u64 f = 0, fs = 0;
   for (u32 i = blockIdx.x * STAT_BS + threadIdx.x; i < ha_p.nsbs; i += STAT_PARTS * STAT_BS) {
     const u32 cs = ld32(&ha_p.desc[i].chunk_sz);
-    const u32 used = cs ? chunk_mul(ctr_count(ld64(ctr_of(i))), cs) : 0u;
+    const u32 used = cs ? chunk_mul(ctr_count(ld64(ctr_of(ha_p, i))), cs) : 0u;
     f += ha_p.sb_sz - used;
     if (cs == 0) fs += ha_p.sb_sz;
   }
