@@ -229,7 +229,9 @@ __device__ __forceinline__ void wave_count(unsigned long long* c, bool hit) {
 // atomics, so the eighth resident wave per SIMD pays.  NULLs and damaged
 // patterns are counted where they happen, so that no per-lane counter stays
 // live through the inlined allocator: with two such counters the 8-wave
-// build spilled 12 VGPRs and ran about 7% slower.
+// build spilled 12 VGPRs and ran about 7% slower.  The read-back is one
+// 16-byte load: left to the short-circuit of the compare, its first word was
+// loaded and awaited before the rest.
 __global__ void __launch_bounds__(256, 8) plain_k(int nthreads, int size, int iters, unsigned long long* errs,
                         unsigned long long* nulls) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -243,7 +245,8 @@ __global__ void __launch_bounds__(256, 8) plain_k(int nthreads, int size, int it
     p[0] = a;
     p[1] = b;
     __asm__ __volatile__("" ::: "memory");
-    const uint2 ra = p[0], rb = p[1];
+    uint2 ra = p[0], rb = p[1];
+    __asm__ __volatile__("" : "+v"(ra.x), "+v"(ra.y), "+v"(rb.x), "+v"(rb.y));  // all read before any compare
     wave_count(errs, ra.x != a.x || ra.y != a.y || rb.x != b.x || rb.y != b.y);
     hafree(p);
   }
@@ -557,14 +560,28 @@ __device__ __forceinline__ void fill_node(NodeHdr* h, u32* a, u32 seed, u32 job,
   h->deg = deg;
   h->adj = a;
 }
-__device__ __forceinline__ u32 check_node(const NodeHdr* h, u32 seed, u32 job, u32 node, u32 n, u32 deg) {
-  if (h->node != node || h->deg != deg || !h->adj) return 1;
+// The header is one 16-byte load, and the pairs are loaded CHECK_PAIRS at a
+// time before any is compared: with one pair awaited after another, a degree
+// of 8 was four round trips to the blocks.
+constexpr u32 CHECK_PAIRS = 4;
+__device__ __forceinline__ u32 check_node(const NodeHdr* h, u32 seed, u32 job, u32 node, u32 n, u32 deg,
+                                          u32*& adj) {
+  const uint4 hv = *(const uint4*)h;
+  adj = (u32*)(((u64)hv.w << 32) | hv.z);
+  if (hv.x != node || hv.y != deg || !adj) return 1;
   const u32 m = ha::mod_magic(n);
   u32 bad = 0;
-  for (u32 e = 0; e < deg; e += 2) {
-    const uint2 v = *(const uint2*)(h->adj + e);
-    bad += v.x != ha::mod_by(gh(seed, job, node, e), n, m);
-    if (e + 1 < deg) bad += v.y != ha::mod_by(gh(seed, job, node, e + 1), n, m);
+  for (u32 e0 = 0; e0 < deg; e0 += 2 * CHECK_PAIRS) {
+    uint2 v[CHECK_PAIRS];
+#pragma unroll
+    for (u32 t = 0; t < CHECK_PAIRS; ++t)
+      v[t] = e0 + 2 * t < deg ? *(const uint2*)(adj + e0 + 2 * t) : make_uint2(0u, 0u);
+#pragma unroll
+    for (u32 t = 0; t < CHECK_PAIRS; ++t) {
+      const u32 e = e0 + 2 * t;
+      if (e < deg) bad |= v[t].x ^ ha::mod_by(gh(seed, job, node, e), n, m);
+      if (e + 1 < deg) bad |= v[t].y ^ ha::mod_by(gh(seed, job, node, e + 1), n, m);
+    }
   }
   return bad ? 1 : 0;
 }
@@ -603,10 +620,11 @@ __global__ void graph_plain_free_k(const u64* offs, const u32* nnodes, u32 njobs
   NodeHdr* h = table[gi];
   if (!h) return;
   const u32 job = job_of(offs, njobs, gi), node = (u32)(gi - offs[job]);
-  if (check_node(h, seed, job, node, nnodes[job], poisson8(seed, job, node))) {
+  u32* adj = nullptr;
+  if (check_node(h, seed, job, node, nnodes[job], poisson8(seed, job, node), adj)) {
     atomicAdd(&stats[1], 1ull);  // a damaged header's adjacency pointer is not trusted
   } else {
-    hafree(h->adj);
+    hafree(adj);
   }
   hafree(h);
 }
