@@ -8,6 +8,7 @@
 //               count bits 32..63, head references 16..23, chunk id 8..11
 //   desc        nsbs Desc: size id, chunk id, chunk size, head references (src/slab.h:16-29)
 //   sb_lock     nsbs u32                                                (src/slab.cuh:18)
+//   full        nsbs u32: the count has reached the busy threshold
 //   sets        NSETS * nsw u64 slab bitmaps: free, roomy[16], busy[16], sparse[4]
 //   head/cached/head_lock/ticket: nheads * 16 u32 each, one per 128 B line
 //   lbits       ceil(lunits/64) u64: one bit per 4 KiB unit of the large region
@@ -84,6 +85,7 @@ struct Params {
   u64* ctr;
   Desc* desc;
   u32* sb_lock;
+  u32* full;        // per slab: its count may be at or above the busy threshold
   u64* sets;
   u32* head;
   u32* cached;

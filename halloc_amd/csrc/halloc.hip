@@ -548,6 +548,7 @@ HA_DEV u32 new_sb_for_size(u32 size_id, u32 ihead, u32 seen, bool force = false)
       u32 nh;
       // below: a forced replacement of a head that still has room
       const bool below = cur != SB_NONE && ctr_count(ul64(ctr_of(P, cur & ~HEAD_EXT))) < head_limit(cur, s);
+      if (below && !(cur & HEAD_EXT) && ul32(P.full + cur)) st32(P.full + cur, 0u);  // an outdated mark
       const u32 fe = ul32(P.free_ep);
       if (below && ul32(fp) == cur && ul32(fp + 1) == fe) {
         nh = cur;  // this head's forced search failed, and no slab became free since
@@ -617,6 +618,16 @@ HA_DEV u32 mod_chunks(const SizeInfo& s, u64 x) {
 // nibbles, and leaves each reserved lane's chunk in my_ich.  itry advances for
 // the whole group; off0 is the probe offset of the first attempt (a run that
 // resumes after a first attempt made elsewhere starts at itry 1).
+// The check that the slab is not full reads the slab's full mark: set by the
+// group whose add reaches the busy threshold, cleared by the free that falls
+// below it, and by a head search that finds it outdated (a race between the
+// two).  Only a head filled further (HEAD_EXT) needs the count itself.
+// Loading the counter at every check put loads and atomics on one line, and
+// where the L2 caches a line that others add to, each waits for the other:
+// 64 words hot at once, an atomic alone took 22 ns a word, with a load beside
+// it 213 ns.  2^20 threads of 8..256 B on 512 MiB, where two counters a class
+// serve the whole chip, took 3.5 ms a launch of four rounds and take 1.5 ms
+// with the mark.
 HA_DEV u64 probe_run(const Params& P_, const SizeInfo& s, u32 hsb, u32 limit, u32 old, u64 P, u32 me, u32& itry, u32& my_ich,
                      u64 off0 = 0, bool* spent = nullptr) {
   const u32 k = s.ncib, nchunks = s.nchunks, nwb = nchunks >> 6, nwn = nchunks >> 4;
@@ -629,9 +640,15 @@ HA_DEV u64 probe_run(const Params& P_, const SizeInfo& s, u32 hsb, u32 limit, u3
   u64* bw = bits_of(P_, hsb);
   u64* nw = nibs_of(P_, hsb);
   u64 reserved = 0;
-  u64 off = off0;
+  // off: the probe offset modulo the slab; hstep: the stride of probe itry
+  // (itry * STEP_FREQ * k modulo hash_step), dstep its growth per probe: both
+  // set at the first probe that fails (dstep is never 0: hash_step is k times
+  // an odd prime)
+  u32 off = mod_chunks(s, off0), hstep = 0, dstep = 0;
   for (;;) {
-    const u32 pA = mod_chunks(s, (u64)runA + off), pB = mod_chunks(s, (u64)runB + off);
+    u32 pA = runA + off, pB = runB + off;  // below 2 * nchunks < 2^32
+    pA = pA >= nchunks ? pA - nchunks : pA;
+    pB = pB >= nchunks ? pB - nchunks : pB;
     const u32 st = inA ? pA + slot0 * k : pB - split * k;
     u32 wb, ib;
     u64 ub;
@@ -647,8 +664,9 @@ HA_DEV u64 probe_run(const Params& P_, const SizeInfo& s, u32 hsb, u32 limit, u3
     const bool ok = inP && !(oldw & mym);
     const u64 S = ballot(ok) & P;  // P: this lane's group (other groups probe alongside)
     const u64 F = P & ~S;
-    if (F) {
-      // give back the bits the failing lanes set (src/slab.cuh:480-483)
+    if (F && k > 1) {
+      // give back the bits the failing lanes set (src/slab.cuh:480-483); a
+      // one-chunk field that fails was taken whole
       u32 wf, iff;
       u64 uf;
       run_word_bits(F & myseg, me, st, k, wf, uf, iff);
@@ -668,14 +686,20 @@ HA_DEV u64 probe_run(const Params& P_, const SizeInfo& s, u32 hsb, u32 limit, u3
     P = F;
     if (!P) break;
     if (itry % CHECK_NTRIES == CHECK_NTRIES - 1) {
-      if (ctr_count(ld64(ctr_of(P_, hsb))) >= limit) break;
+      if (rfl(ld32(P_.full + hsb)) && (limit == s.busy_thr || ctr_count(ld64(ctr_of(P_, hsb))) >= limit)) break;
     }
-    const u32 step = mod_by((itry + 1) * STEP_FREQ * k, s.hash_step, s.hash_step_m);
-    off = (u64)(itry + 1) * step;
     if (++itry % MAX_NTRIES >= MAX_NTRIES - 1) {
       if (spent) *spent = true;
       break;
     }
+    if (dstep == 0) {
+      dstep = mod_by(STEP_FREQ * k, s.hash_step, s.hash_step_m);
+      hstep = mod_by(itry * STEP_FREQ * k, s.hash_step, s.hash_step_m);
+    } else {
+      hstep += dstep;
+      hstep = hstep >= s.hash_step ? hstep - s.hash_step : hstep;
+    }
+    off = mod_chunks(s, (u64)itry * hstep);
   }
   return reserved;
 }
@@ -737,6 +761,7 @@ HA_DEV void* malloc_group(u32 sid, u64 g, u32 ihead, u32 me) {
           need = true;
         } else {
           const u32 oc = ctr_count(oldc);
+          if (oc < s.busy_thr && oc + change >= s.busy_thr && me == lead) st32(P.full + hsb, 1u);
           if (oc < limit && oc + change >= limit) need = true;
           if (mine) p = slab_of(P, hsb) + chunk_mul(my_ich, s.chunk_sz);
           want &= ~reserved;
@@ -882,6 +907,7 @@ HA_DEV void malloc_batch_group(u32 sid, u64 g, u32 ihead, u32 me, u32 cnt, void*
         need = true;
       } else {
         const u32 oc = ctr_count(oldc);
+        if (oc < s.busy_thr && oc + change >= s.busy_thr && me == lead) st32(P_.full + hsb, 1u);
         if (oc < limit && oc + change >= limit) need = true;
       }
     }
@@ -910,6 +936,11 @@ HA_DEV void* malloc_small(u32 nbytes, u32 ihead) {
 }
 
 // --------------------------------------------------------------- free path
+// a decrement from oc to nc that takes the slab below its busy threshold
+HA_DEV void unmark_full(const Params& P, u32 sb, u32 oc, u32 nc, u32 busy_thr) {
+  if (oc >= busy_thr && nc < busy_thr) st32(P.full + sb, 0u);
+}
+
 // hafree_small (src/halloc.cu:211-230) for NR rounds at once: in round j the
 // lanes with act[j] free the block at arena offset off[j].  The slab
 // descriptors of every round are loaded together, then every round's
@@ -941,6 +972,7 @@ HA_DEV void free_rounds(const u64* off, const bool* act) {
       cs[j] = cid[j] == SZ_NONE ? 0u : ((cid[j] & 1) ? 3u << 16 | 3u : 1u << 16 | 4u) + (cid[j] >> 1) * 4u;
     }
   }
+  u32 thr[NR];  // the slab's busy threshold, for unmark_full
   // nibbles: read back the block lengths and clear them
   u32 ich[NR], nch[NR], k[NR], st[NR];
   u64 A[NR], myseg[NR], o[NR];
@@ -956,6 +988,8 @@ HA_DEV void free_rounds(const u64* off, const bool* act) {
     myseg[j] = o[j] = 0;
     inn[j] = 64;
     fast[j] = false;
+    thr[j] = ~0u;
+    bool one = false;  // every block in one slab
     // fast path: the lanes free one slab's blocks laid out as at most two runs
     // (what one class group of a wave allocates): one atomic per word touched
     if (A[j]) {
@@ -963,8 +997,10 @@ HA_DEV void free_rounds(const u64* off, const bool* act) {
       const u32 sb0 = rdl(sb[j], l0);
       if (ballot(valid && sb[j] == sb0) == A[j]) {
         const u32 sid0 = rdl(sid[j], l0);
+        one = true;
         if (sid0 < NSIZES) {
           k[j] = P.si[sid0].ncib;
+          thr[j] = P.si[sid0].busy_thr;
           const u32 sa = rdl(ich[j], l0) - l0 * k[j];
           const bool ina = valid && ich[j] == sa + me * k[j];
           const u64 Am = ballot(ina);
@@ -985,6 +1021,8 @@ HA_DEV void free_rounds(const u64* off, const bool* act) {
         }
       }
     }
+    // several slabs: each lane's own, loaded here to arrive with the nibbles
+    if (!one && sid[j] < NSIZES) thr[j] = P.si[sid[j]].busy_thr;
     u64* nw = nibs_of(P, sb[j]);
     if (fast[j]) {
       u32 wn;
@@ -998,6 +1036,7 @@ HA_DEV void free_rounds(const u64* off, const bool* act) {
   // bits
 #pragma unroll
   for (int j = 0; j < NR; ++j) {
+    __asm__ volatile("" : "+v"(thr[j]));
     const bool valid = act[j] && cs[j] != 0;
     u64* bw = bits_of(P, sb[j]);
     if (fast[j]) {
@@ -1053,9 +1092,10 @@ HA_DEV void free_rounds(const u64* off, const bool* act) {
   }
 #pragma unroll
   for (int j = 0; j < NR; ++j) {
+    const u32 oc = ctr_count(oldc[j]), nc = oc - change[j];
+    if (lead[j]) unmark_full(P, sb[j], oc, nc, thr[j]);
     const bool tr = lead[j] && !ctr_is_head(oldc[j]) && sid[j] < NSIZES && cid[j] != SZ_NONE &&
-                    sb_class(ctr_count(oldc[j]), P.si[sid[j]]) !=
-                        sb_class(ctr_count(oldc[j]) - change[j], P.si[sid[j]]);
+                    sb_class(oc, P.si[sid[j]]) != sb_class(nc, P.si[sid[j]]);
     u64 T = ballot(tr);
     while (T) {
       const u32 l = (u32)__builtin_ctzll(T);
@@ -1185,9 +1225,11 @@ HA_DEV void free_runs(u32 F, RunRounds r) {
     if (me == l) tot = acc;
     rem &= ~G;
   }
+  const u32 thr = inF && rsid < NSIZES ? P.si[rsid].busy_thr : ~0u;
   u64 told = 0;
   if (inF && me == ldr) told = a_sub(ctr_of(P, rsb), (u64)tot << CTR_COUNT_SH);
   const u64 oldc = shfl64(told, ldr) - ((u64)pre << CTR_COUNT_SH);
+  if (inF) unmark_full(P, rsb, ctr_count(oldc), ctr_count(oldc) - rch, thr);
   const bool tr = inF && !ctr_is_head(oldc) && rsid < NSIZES && rcid != SZ_NONE &&
                   sb_class(ctr_count(oldc), P.si[rsid < NSIZES ? rsid : 0]) !=
                       sb_class(ctr_count(oldc) - rch, P.si[rsid < NSIZES ? rsid : 0]);
@@ -1760,6 +1802,7 @@ static int init_locked(const ha_opts_c& o) {
   u64 o_nibs = off; off = align_up(off + (u64)P.nsbs * P.nib_words * 8, 256);
   u64 o_ctr = off; off = align_up(off + (u64)P.nsbs * CTR_STRIDE * 8, 256);
   u64 o_desc = off; off = align_up(off + (u64)P.nsbs * sizeof(Desc), 256);
+  u64 o_full = off; off = align_up(off + (u64)P.nsbs * 4, 256);
   u64 o_lock = off; off = align_up(off + (u64)P.nsbs * 4, 256);
   u64 o_sets = off; off = align_up(off + (u64)NSETS * P.nsw * 8, 256);
   u64 hot_bytes = (u64)P.nheads * NSIZES * HOT_STRIDE * 4;
@@ -1791,6 +1834,7 @@ static int init_locked(const ha_opts_c& o) {
   P.nibs = (u64*)(m + o_nibs);
   P.ctr = (u64*)(m + o_ctr);
   P.desc = (Desc*)(m + o_desc);
+  P.full = (u32*)(m + o_full);
   P.sb_lock = (u32*)(m + o_lock);
   P.sets = (u64*)(m + o_sets);
   P.head = (u32*)(m + o_head);

@@ -81,3 +81,40 @@ def test_batched_free_of_a_partial_wave(heap, which):
     d = H.Halloc.dump()
     assert (d == m.dump()).all()
     assert ((d[:H.Halloc.geometry()["nsbs"]] >> np.uint64(32)) == 0).all()
+
+
+def refill_program(sizes, nsteps, keep, seed):
+    """One wave of mixed sizes from `sizes`, freeing a share of the live blocks
+    that alternates between (1 - keep) and keep of the allocations, so that
+    slabs pass their busy threshold in both directions again and again."""
+    rng = np.random.default_rng(seed)
+    ops = np.zeros((nsteps, 64, 2), dtype=np.uint32)
+    live = []
+    for st in range(nsteps):
+        p = keep if (st // 20) % 2 else 1 - keep
+        for l in range(64):
+            if live and rng.random() < p:
+                ops[st, l] = (2, live.pop(int(rng.integers(len(live)))))
+            else:
+                ops[st, l] = (1, int(rng.choice(sizes)))
+        live.extend(st * 64 + l for l in range(64) if ops[st, l, 0] == 1)
+    return ops
+
+
+@pytest.mark.parametrize("nheads,memory,sizes", [(1, 16 << 20, (700, 1500, 3000, 100, 200)), (1, 12 << 20, (3072,)),
+                                                 (1, 12 << 20, (256, 384)), (1, 12 << 20, (16, 24)), (1, 12 << 20, (128, 192)),
+                                                 (8, 40 << 20, (700, 1500, 3000, 100, 200))])
+def test_heads_pass_the_busy_threshold_both_ways(heap, nheads, memory, sizes):
+    # full heads, shared heads, heads filled past the threshold and exhaustion:
+    # records and state equal the host model's bit for bit
+    from oracle import model as M
+    print(f"[gpu] busy threshold nheads={nheads} sizes={sizes}", flush=True)
+    heap(H.HallocOpts(memory=memory, sb_sz_sh=21, nheads=nheads))
+    nh = H.Halloc.geometry()["nheads"]
+    ops = refill_program(sizes, 240, 0.3, 11)
+    ih = np.arange(240, dtype=np.uint32) % nh
+    recs, _ = H.Halloc.replay(ops, ih)
+    m = M.ModelHeap(M.make_opts(memory=memory, sb_sz_sh=21, nheads=nheads, hash_mode=1))
+    want, _ = m.replay(ops, ih)
+    assert (recs == want).all()
+    assert (H.Halloc.dump() == m.dump()).all()
