@@ -118,3 +118,22 @@ def test_heads_pass_the_busy_threshold_both_ways(heap, nheads, memory, sizes):
     want, _ = m.replay(ops, ih)
     assert (recs == want).all()
     assert (H.Halloc.dump() == m.dump()).all()
+
+
+@pytest.mark.parametrize("length", [1, 15, 16, 17, 33, 64])
+@pytest.mark.parametrize("nreq", [1, 3, 64, 256, 700])
+def test_pages_drained_together(heap, nreq, length):
+    # equal lengths that arrive together: up to 64 lanes of a wave drain in the
+    # same step (the shared check takes four pages at a time), last pages part
+    # filled; in the mixed run lengths vary by lane
+    from halloc_amd.workloads import pages_for
+    from tests.helpers import serve_checksums
+    print(f"[gpu] drain nreq={nreq} length={length}", flush=True)
+    heap(H.HallocOpts(memory=64 << 20, sb_sz_sh=21, nheads=8))
+    rng = np.random.default_rng(nreq * 100 + length)
+    tag = rng.integers(0, 1 << 32, nreq, dtype=np.uint64).astype(np.uint32)
+    for ln in (np.full(nreq, length, np.uint32), rng.integers(1, length + 1, nreq).astype(np.uint32)):
+        r = H.Halloc.run_serve(np.zeros(nreq, np.uint64), ln, tag, slots=256, watermark=0)
+        assert r["completed"] == nreq and r["nulls"] == 0 and not r["bad"].any()
+        assert (r["produced"] == ln).all() and (r["checksum"] == serve_checksums(tag, ln)).all()
+        assert r["pages"] == int(pages_for(ln).sum())
