@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -1594,6 +1595,13 @@ int fail(int code, const std::string& msg) {
     if (e_ != hipSuccess) return ::ha::fail(HA_E_HIP, std::string(#call) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
+// What init and shutdown call so that memory kept elsewhere is given back.
+static std::atomic<void (*)()> g_release{nullptr};
+void on_release(void (*f)()) { g_release = f; }
+static void release_kept() {
+  if (auto f = g_release.load()) f();
+}
+
 // Uncached arenas are never freed once a kernel has touched them (freeing
 // such memory has corrupted later allocations on this platform); shutdown
 // hands the arena back to this pool and a later init on the same device
@@ -1718,6 +1726,7 @@ static int scratch_ptr(u64** out);
 static int g_heap_dev = -1;  // the device ha_init initialized
 
 static int shutdown_locked() {
+  release_kept();
   if (!g_host.initialized) return HA_OK;
   Params zero;
   std::memset(&zero, 0, sizeof zero);
@@ -1732,10 +1741,7 @@ static int shutdown_locked() {
 }
 
 static int init_locked(const ha_opts_c& o) {
-  if (g_host.initialized) {
-    int rc = shutdown_locked();
-    if (rc) return rc;
-  }
+  if (int rc = shutdown_locked()) return rc;
   if (o.sb_sz_sh < (int)MIN_SB_SZ_SH || o.sb_sz_sh > (int)MAX_SB_SZ_SH)
     return fail(HA_E_INVALID, "sb_sz_sh must be in 21..26");
   if (o.nheads < 0 || o.nheads > (int)MAX_NHEADS) return fail(HA_E_INVALID, "nheads must be in 0..64");

@@ -137,3 +137,41 @@ def test_pages_drained_together(heap, nreq, length):
         assert r["completed"] == nreq and r["nulls"] == 0 and not r["bad"].any()
         assert (r["produced"] == ln).all() and (r["checksum"] == serve_checksums(tag, ln)).all()
         assert r["pages"] == int(pages_for(ln).sum())
+
+
+@pytest.mark.parametrize("nthreads", [1, 4])
+def test_buffers_kept_between_calls(heap, nthreads):
+    # calls of changing sizes, from several threads, with a refused call between:
+    # every call sees its own values, also after a shutdown and a new heap
+    import threading
+
+    print(f"[gpu] kept buffers threads={nthreads}", flush=True)
+    opts = H.HallocOpts(memory=256 << 20, sb_sz_sh=21, nheads=8)
+    wrong = []
+
+    def calls(t):
+        try:
+            rng = np.random.default_rng(t)
+            for n in (1, 1000, 70, 30000, 1, 4097, 30000, 200):
+                sizes = rng.integers(1, 257, (3, n)).astype(np.uint32)
+                order = rng.permutation(3 * n).astype(np.uint32)
+                r = H.Halloc.run_lists(sizes, order, bs=64)
+                assert r["requests"] == 3 * n and r["nulls"] == 0 and r["errors"] == 0
+                with pytest.raises(H.HallocError):
+                    H.Halloc.run_lists(sizes, np.zeros(3 * n, np.uint32), bs=64)
+                p = H.Halloc.malloc_sizes(sizes[0])
+                assert (p != 0).all() and len(np.unique(p)) == n
+                H.Halloc.free_ptrs(p)
+        except BaseException as e:  # reported below: a thread's own failure would be lost
+            wrong.append(repr(e))
+
+    for _ in range(2):
+        heap(opts)
+        ths = [threading.Thread(target=calls, args=(t,)) for t in range(nthreads)]
+        for th in ths:
+            th.start()
+        for th in ths:
+            th.join()
+        assert not wrong
+        assert H.Halloc.free_bytes() == H.Halloc.geometry()["arena_bytes"]
+        H.Halloc.shutdown()
