@@ -732,21 +732,12 @@ __device__ __forceinline__ u32 check_node(const NodeHdr* h, u32 seed, u32 job, u
   }
   return bad ? 1 : 0;
 }
-__device__ __forceinline__ u32 job_of(const u64* offs, u32 njobs, u64 gi) {
-  u32 lo = 0, hi = njobs;  // offs[lo] <= gi < offs[hi]
-  while (hi - lo > 1) {
-    u32 mid = (lo + hi) / 2;
-    if (offs[mid] <= gi) lo = mid; else hi = mid;
-  }
-  return lo;
-}
-
 // plain per-call form: one thread per node of the job range [j0, j1)
 __global__ void graph_plain_build_k(const u64* offs, const u32* nnodes, u32 njobs, u32 seed, u64 g0, u64 g1,
                                     NodeHdr** table, unsigned long long* stats) {
   const u64 gi = g0 + blockIdx.x * (u64)blockDim.x + threadIdx.x;
   if (gi >= g1) return;
-  const u32 job = job_of(offs, njobs, gi), node = (u32)(gi - offs[job]), n = nnodes[job];
+  const u32 job = ha::job_at(offs, njobs, gi), node = (u32)(gi - offs[job]), n = nnodes[job];
   const u32 deg = poisson8(seed, job, node);
   NodeHdr* h = (NodeHdr*)hamalloc(sizeof(NodeHdr));
   u32* a = (u32*)hamalloc(adj_bytes(deg));
@@ -766,7 +757,7 @@ __global__ void graph_plain_free_k(const u64* offs, const u32* nnodes, u32 njobs
   if (gi >= g1) return;
   NodeHdr* h = table[gi];
   if (!h) return;
-  const u32 job = job_of(offs, njobs, gi), node = (u32)(gi - offs[job]);
+  const u32 job = ha::job_at(offs, njobs, gi), node = (u32)(gi - offs[job]);
   u32* adj = nullptr;
   if (check_node(h, seed, job, node, nnodes[job], poisson8(seed, job, node), adj)) {
     atomicAdd(&stats[1], 1ull);  // a damaged header's adjacency pointer is not trusted
@@ -792,6 +783,17 @@ __global__ void graph_reset_k(u32* next, u32* built, u32 njobs) {
   const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i == 0) *next = 0;
   for (u32 k = i; k < njobs; k += gridDim.x * blockDim.x) built[k] = 0;
+}
+
+// The batched form's item sequence, one thread per chunk; a few us, bound by the
+// dependent loads of two binary searches.  Built on the host and copied, it was
+// 0.25 ms and more of a call over 1024 jobs (the call 2.65 -> 2.43 ms).
+__global__ void graph_seq_k(const u32* coffs, u32 njobs, u64 lag, u64* seq) {
+  const u32 b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= coffs[njobs]) return;
+  const ha::GraphItem g = ha::graph_item(coffs, njobs, lag, b);
+  seq[g.build_at] = g.item;
+  seq[g.free_at] = g.item | ha::GRAPH_FREE_ITEM;
 }
 
 __device__ __forceinline__ u32 rfl32(u32 v) { return (u32)__builtin_amdgcn_readfirstlane((int)v); }
@@ -2786,33 +2788,16 @@ int ha_run_graphs(const ha_graph_args* a, const uint32_t* nnodes, ha_graph_resul
   std::vector<u32> coffs(njobs + 1, 0);
   for (u32 j = 0; j < njobs; ++j) coffs[j + 1] = coffs[j] + (nnodes[j] + per_chunk - 1) / per_chunk;
   const u32 nitems = coffs[njobs];
-  // the item sequence: builds in job order, each job's frees `lag` items after its last build
-  const u64 lag = (u64)a->waves * GRAPH_GRAB;
-  std::vector<u64> seq;
-  seq.reserve(2 * (size_t)nitems);
-  u32 jf = 0;  // next job whose frees are due
-  for (u64 b = 0; b < (u64)nitems + lag; ++b) {
-    if (b < nitems) {
-      const u32 j = (u32)(std::upper_bound(coffs.begin(), coffs.end(), (u32)b) - coffs.begin()) - 1;
-      seq.push_back(((u64)j << 32) | (b - coffs[j]));
-    }
-    while (jf < njobs && (u64)coffs[jf + 1] - 1 + lag <= b) {
-      for (u32 c = 0; c < coffs[jf + 1] - coffs[jf]; ++c) seq.push_back((1ull << 63) | ((u64)jf << 32) | c);
-      ++jf;
-    }
-  }
-  while (jf < njobs) {
-    for (u32 c = 0; c < coffs[jf + 1] - coffs[jf]; ++c) seq.push_back((1ull << 63) | ((u64)jf << 32) | c);
-    ++jf;
-  }
-  const u32 nseq = (u32)seq.size();
+  const u64 lag = (u64)a->waves * GRAPH_GRAB;  // a job's frees come this many items after its last build
+  const u32 nseq = 2 * nitems;
   DBuf dcoffs, dseq, dnext, dbuilt;
   HH(dcoffs.alloc((njobs + 1) * 4));
   HH(dseq.alloc((size_t)nseq * 8));
   HH(dnext.alloc(4));
   HH(dbuilt.alloc(njobs * 4));
   HH(hipMemcpy(dcoffs.p, coffs.data(), (njobs + 1) * 4, hipMemcpyHostToDevice));
-  HH(hipMemcpy(dseq.p, seq.data(), (size_t)nseq * 8, hipMemcpyHostToDevice));
+  graph_seq_k<<<(nitems + 255) / 256, 256, 0, s.s>>>((const u32*)dcoffs.p, njobs, lag, (u64*)dseq.p);
+  HH(hipGetLastError());
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   const unsigned bgrid = (unsigned)((a->waves * 64 + 255) / 256);
@@ -2842,7 +2827,7 @@ int ha_run_graphs(const ha_graph_args* a, const uint32_t* nnodes, ha_graph_resul
       nch[j] = coffs[j + 1] - coffs[j];
       for (u32 c = 0; c < nch[j]; ++c) {
         sb.push_back(((u64)j << 32) | c);
-        sf.push_back((1ull << 63) | ((u64)j << 32) | c);
+        sf.push_back(ha::GRAPH_FREE_ITEM | ((u64)j << 32) | c);
       }
     }
     // the batched kernel over `items`; preset: every job's build count starts complete

@@ -34,3 +34,12 @@ def test_poisson8_table_matches_scipy(tmp_path):
     deg = np.searchsorted(t, u, side="right")
     hist = np.bincount(deg, minlength=len(t)) / len(u)
     assert np.abs(hist[:30] - poisson.pmf(np.arange(30), 8)).max() < 1e-4
+
+
+def test_graph_item_sequence(tmp_path):
+    exe = tmp_path / "graph_seq_check"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-o", str(exe),
+                    os.path.join(HERE, "native", "graph_seq_check.cpp")], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert r.stdout.strip() == "ok"
