@@ -175,3 +175,27 @@ def test_buffers_kept_between_calls(heap, nthreads):
         assert not wrong
         assert H.Halloc.free_bytes() == H.Halloc.geometry()["arena_bytes"]
         H.Halloc.shutdown()
+
+
+@pytest.mark.parametrize("n,per", [(1, 1), ((1 << 17) - 1, 1), (1 << 16, 2), (43691, 3), (1 << 17, 1), (100003, 7)])
+def test_list_orders_checked(heap, n, per):
+    # below, at and above the length from which the device checks the order and
+    # counts the requests: permutations are taken, anything else is refused
+    # before a block is allocated
+    print(f"[gpu] list order n={n} per={per}", flush=True)
+    heap(H.HallocOpts(memory=256 << 20, sb_sz_sh=22))
+    total = n * per
+    rng = np.random.default_rng(total)
+    sizes = (rng.integers(0, 3, (per, n)) * 16).astype(np.uint32)
+    good = rng.permutation(total).astype(np.uint32)
+    for order in (None, good, np.arange(total, dtype=np.uint32), np.arange(total, dtype=np.uint32)[::-1]):
+        r = H.Halloc.run_lists(sizes, order)
+        assert r["requests"] == np.count_nonzero(sizes) and r["nulls"] == 0 and r["errors"] == 0
+    arena = H.Halloc.geometry()["arena_bytes"]
+    for k in (0, total // 2, total - 1):
+        for v in (total, 0xFFFFFFFF, int(good[k - 1]) if total > 1 else total + 1):
+            bad = good.copy()
+            bad[k] = v
+            with pytest.raises(H.HallocError, match="permutation"):
+                H.Halloc.run_lists(sizes, bad)
+    assert H.Halloc.free_bytes() == arena
