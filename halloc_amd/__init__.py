@@ -32,7 +32,7 @@ EXPORTS = ("ha_default_opts", "ha_init_c", "ha_shutdown_c", "ha_extfrag_c", "ha_
            "ha_run_plain", "ha_malloc_sizes", "ha_free_ptrs", "ha_read_words", "ha_probe_atomics",
            "ha_run_lists", "ha_run_phase", "ha_replay_batch", "ha_run_graphs", "ha_run_serve",
            "ha_probe_copy", "ha_run_test", "ha_run_sample", "ha_run_corr_test0", "ha_probe_chain",
-           "ha_free_bytes_noalloc_c", "ha_run_touch")
+           "ha_free_bytes_noalloc_c", "ha_run_touch", "ha_full_marks")
 
 
 class HallocError(RuntimeError):
@@ -196,6 +196,7 @@ def lib() -> ctypes.CDLL:
         "ha_replay": (i32, [vp, i32, i32, vp, vp, vp]),
         "ha_dump_words": (ctypes.c_int64, []),
         "ha_dump": (i32, [vp, ctypes.c_int64]),
+        "ha_full_marks": (i32, [vp, ctypes.c_int64]),
         "ha_run_plain": (i32, [i32, i32, i32, i32, i32, i32, vp, P(_PlainResult)]),
         "ha_malloc_sizes": (i32, [vp, i32, i32, vp]),
         "ha_run_corr_test0": (i32, [i32, i32, i32, P(_Corr0Result)]),
@@ -300,6 +301,13 @@ class Halloc:
         n = _check(lib().ha_dump_words())
         out = np.zeros(n, dtype=np.uint64)
         _check(lib().ha_dump(out.ctypes.data, n))
+        return out
+
+    @staticmethod
+    def full_marks() -> np.ndarray:
+        """The slabs' full marks (uint32, one per slab)."""
+        out = np.zeros(Halloc.geometry()["nsbs"], dtype=np.uint32)
+        _check(lib().ha_full_marks(out.ctypes.data, out.size))
         return out
 
     @staticmethod

@@ -33,6 +33,7 @@
 #include "../../include/halloc.h"
 #include "../../include/halloc_amd.h"
 #include "ha_internal.h"
+#include "ha_mark.h"
 
 namespace ha {
 
@@ -118,6 +119,21 @@ HA_DEV u64* nibs_of(const Params& P, u32 sb) { return P.nibs + ((u64)sb << (P.sb
 HA_DEV char* slab_of(const Params& P, u32 sb) { return P.arena + ((u64)sb << P.sb_sz_sh); }
 HA_DEV u32* hot(u32* base, u32 ihead, u32 sid) { return base + (ihead * NSIZES + sid) * HOT_STRIDE; }
 HA_DEV u64* set_words(const Params& P, u32 set) { return P.sets + (u64)set * P.nsw; }
+
+// a slab's full mark (ha_mark.h); settle() waits for the store's completion at
+// the device, without the write-back and invalidation of a fence
+struct SlabMark {
+  const Params& P;
+  u32 sb;
+  HA_DEV void set(u32 v) const { st32(P.full + sb, v); }
+  HA_DEV u32 get() const { return ld32(P.full + sb); }
+  HA_DEV void settle() const { __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+  HA_DEV bool full() const {
+    const u32 sid = ld32(&P.desc[sb].size_id);
+    return sid < NSIZES && ctr_count(ld64(ctr_of(P, sb))) >= P.si[sid].busy_thr;
+  }
+};
+HA_DEV SlabMark mark_of(const Params& P, u32 sb) { return SlabMark{P, sb}; }
 
 // ----------------------------------------------------- single-lane slow path
 // Everything below until malloc_group runs on exactly one lane of a wave.
@@ -214,6 +230,15 @@ HA_DEV void ctr_transitions(u32 sb, u64 old, u32 change) {
   }
 }
 
+// a group gave back the `change` chunks it had added to a slab that had passed
+// to another class: `old` is the counter before it did
+HA_DEV void add_taken_back(u32 sb, u64 old, u32 change) {
+  const Params& P = params();
+  const u32 size_id = ul32(&P.desc[rfl(sb)].size_id);
+  const u32 oc = ctr_count(rfl64(old));
+  if (size_id < NSIZES) mark_taken_back(mark_of(P, rfl(sb)), oc, oc - rfl(change), P.si[size_id].busy_thr);
+  ctr_transitions(sb, old, change);
+}
 
 // drop one head reference (detach_head, src/slab.cuh:227-255); the last one
 // files the slab by its count.  Caller holds sb_lock[sb].  True if the slab
@@ -548,8 +573,9 @@ HA_DEV u32 new_sb_for_size(u32 size_id, u32 ihead, u32 seen, bool force = false)
       cur = ul32(hp);
       u32 nh;
       // below: a forced replacement of a head that still has room
-      const bool below = cur != SB_NONE && ctr_count(ul64(ctr_of(P, cur & ~HEAD_EXT))) < head_limit(cur, s);
-      if (below && !(cur & HEAD_EXT) && ul32(P.full + cur)) st32(P.full + cur, 0u);  // an outdated mark
+      const u32 cnt = cur != SB_NONE ? ctr_count(ul64(ctr_of(P, cur & ~HEAD_EXT))) : 0u;
+      const bool below = cur != SB_NONE && cnt < head_limit(cur, s);
+      if (cur != SB_NONE) mark_checked(mark_of(P, cur & ~HEAD_EXT), cnt, s.busy_thr);
       const u32 fe = ul32(P.free_ep);
       if (below && ul32(fp) == cur && ul32(fp + 1) == fe) {
         nh = cur;  // this head's forced search failed, and no slab became free since
@@ -619,10 +645,10 @@ HA_DEV u32 mod_chunks(const SizeInfo& s, u64 x) {
 // nibbles, and leaves each reserved lane's chunk in my_ich.  itry advances for
 // the whole group; off0 is the probe offset of the first attempt (a run that
 // resumes after a first attempt made elsewhere starts at itry 1).
-// The check that the slab is not full reads the slab's full mark: set by the
-// group whose add reaches the busy threshold, cleared by the free that falls
-// below it, and by a head search that finds it outdated (a race between the
-// two).  Only a head filled further (HEAD_EXT) needs the count itself.
+// The check that the slab is not full reads the slab's full mark (ha_mark.h):
+// an ordinary head whose mark is set is at its limit; a head filled further
+// (HEAD_EXT) that is marked is looked up in the counter; one that is not
+// marked is below the busy threshold and is probed on, whichever it is.
 // Loading the counter at every check put loads and atomics on one line, and
 // where the L2 caches a line that others add to, each waits for the other:
 // 64 words hot at once, an atomic alone took 22 ns a word, with a load beside
@@ -757,12 +783,12 @@ HA_DEV void* malloc_group(u32 sid, u64 g, u32 ihead, u32 me) {
           if (mine) release_block(hsb, my_ich, k);
           if (me == lead) {
             u64 o = a_sub(ctr_of(P, hsb), (u64)change << CTR_COUNT_SH);
-            ctr_transitions(hsb, o, change);
+            add_taken_back(hsb, o, change);
           }
           need = true;
         } else {
           const u32 oc = ctr_count(oldc);
-          if (oc < s.busy_thr && oc + change >= s.busy_thr && me == lead) st32(P.full + hsb, 1u);
+          if (me == lead) mark_added(mark_of(P, hsb), oc, oc + change, s.busy_thr);
           if (oc < limit && oc + change >= limit) need = true;
           if (mine) p = slab_of(P, hsb) + chunk_mul(my_ich, s.chunk_sz);
           want &= ~reserved;
@@ -903,12 +929,12 @@ HA_DEV void malloc_batch_group(u32 sid, u64 g, u32 ihead, u32 me, u32 cnt, void*
         }
         if (me == lead) {
           u64 o = a_sub(ctr_of(P_, hsb), (u64)change << CTR_COUNT_SH);
-          ctr_transitions(hsb, o, change);
+          add_taken_back(hsb, o, change);
         }
         need = true;
       } else {
         const u32 oc = ctr_count(oldc);
-        if (oc < s.busy_thr && oc + change >= s.busy_thr && me == lead) st32(P_.full + hsb, 1u);
+        if (me == lead) mark_added(mark_of(P_, hsb), oc, oc + change, s.busy_thr);
         if (oc < limit && oc + change >= limit) need = true;
       }
     }
@@ -937,11 +963,6 @@ HA_DEV void* malloc_small(u32 nbytes, u32 ihead) {
 }
 
 // --------------------------------------------------------------- free path
-// a decrement from oc to nc that takes the slab below its busy threshold
-HA_DEV void unmark_full(const Params& P, u32 sb, u32 oc, u32 nc, u32 busy_thr) {
-  if (oc >= busy_thr && nc < busy_thr) st32(P.full + sb, 0u);
-}
-
 // hafree_small (src/halloc.cu:211-230) for NR rounds at once: in round j the
 // lanes with act[j] free the block at arena offset off[j].  The slab
 // descriptors of every round are loaded together, then every round's
@@ -973,7 +994,7 @@ HA_DEV void free_rounds(const u64* off, const bool* act) {
       cs[j] = cid[j] == SZ_NONE ? 0u : ((cid[j] & 1) ? 3u << 16 | 3u : 1u << 16 | 4u) + (cid[j] >> 1) * 4u;
     }
   }
-  u32 thr[NR];  // the slab's busy threshold, for unmark_full
+  u32 thr[NR];  // the slab's busy threshold, for mark_freed
   // nibbles: read back the block lengths and clear them
   u32 ich[NR], nch[NR], k[NR], st[NR];
   u64 A[NR], myseg[NR], o[NR];
@@ -1094,7 +1115,7 @@ HA_DEV void free_rounds(const u64* off, const bool* act) {
 #pragma unroll
   for (int j = 0; j < NR; ++j) {
     const u32 oc = ctr_count(oldc[j]), nc = oc - change[j];
-    if (lead[j]) unmark_full(P, sb[j], oc, nc, thr[j]);
+    if (lead[j]) mark_freed(mark_of(P, sb[j]), oc, nc, thr[j]);
     const bool tr = lead[j] && !ctr_is_head(oldc[j]) && sid[j] < NSIZES && cid[j] != SZ_NONE &&
                     sb_class(oc, P.si[sid[j]]) != sb_class(nc, P.si[sid[j]]);
     u64 T = ballot(tr);
@@ -1230,7 +1251,7 @@ HA_DEV void free_runs(u32 F, RunRounds r) {
   u64 told = 0;
   if (inF && me == ldr) told = a_sub(ctr_of(P, rsb), (u64)tot << CTR_COUNT_SH);
   const u64 oldc = shfl64(told, ldr) - ((u64)pre << CTR_COUNT_SH);
-  if (inF) unmark_full(P, rsb, ctr_count(oldc), ctr_count(oldc) - rch, thr);
+  if (inF) mark_freed(mark_of(P, rsb), ctr_count(oldc), ctr_count(oldc) - rch, thr);
   const bool tr = inF && !ctr_is_head(oldc) && rsid < NSIZES && rcid != SZ_NONE &&
                   sb_class(ctr_count(oldc), P.si[rsid < NSIZES ? rsid : 0]) !=
                       sb_class(ctr_count(oldc) - rch, P.si[rsid < NSIZES ? rsid : 0]);

@@ -2020,6 +2020,15 @@ int ha_dump(uint64_t* out, int64_t nwords) {
   return HA_OK;
 }
 
+int ha_full_marks(uint32_t* out, int64_t nslabs) {
+  const ha::Params& P = ha::host_params();
+  if (!P.initialized) return hfail(HA_E_STATE, "allocator not initialized");
+  if (!out || nslabs < (int64_t)P.nsbs) return hfail(HA_E_INVALID, "mark buffer too small");
+  HH(hipDeviceSynchronize());
+  HH(hipMemcpy(out, P.full, (size_t)P.nsbs * 4, hipMemcpyDeviceToHost));
+  return HA_OK;
+}
+
 int ha_run_plain(int nthreads, int bs, int size, int iters, int warmup, int launches, float* ms,
                  ha_plain_result* res) {
   if (!ha::host_params().initialized) return hfail(HA_E_STATE, "allocator not initialized");

@@ -130,6 +130,11 @@ int ha_replay_batch(const uint32_t *ops, int nsteps, int lanes, uint32_t *recs, 
 int64_t ha_dump_words(void);
 int ha_dump(uint64_t *out, int64_t nwords);
 
+/* The slabs' full marks (one word per slab, not part of the state dump: the
+   host model has none).  With no kernel running, a slab whose count is at its
+   class's busy threshold is marked; a mark on a slab below it is harmless. */
+int ha_full_marks(uint32_t *out, int64_t nslabs);
+
 /* Plain 16 B throughput (tst/perf/priv-throughput/priv-throughput.cu:14-27):
    nthreads lanes in blocks of bs (at most 256); each lane does iters x { p = hamalloc(size);
    write a 16 B pattern {tid, ~tid, tid ^ 0x9E3779B9, iter}; read it back;

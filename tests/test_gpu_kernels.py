@@ -120,6 +120,50 @@ def test_heads_pass_the_busy_threshold_both_ways(heap, nheads, memory, sizes):
     assert (H.Halloc.dump() == m.dump()).all()
 
 
+def unmarked_full_slabs():
+    """Slabs whose count is at their class's busy threshold and whose mark is not set."""
+    g, d, marks = H.Halloc.geometry(), H.Halloc.dump(), H.Halloc.full_marks()
+    n = g["nsbs"]
+    count = (d[:n] >> np.uint64(32)).astype(np.int64)
+    size_id = (d[n:3 * n:2] & np.uint64(0xFFFFFFFF)).astype(np.int64)
+    busy = np.append(np.array(g["size_table"])[:, H.SIZE_TABLE_FIELDS.index("busy")].astype(np.int64), 1 << 40)
+    full = count >= busy[np.minimum(size_id, H.NSIZES)]
+    return int(full.sum()), np.nonzero(full & (marks == 0))[0].tolist()
+
+
+# sizes of one chunk size each: 16, 24, 256 and 384 B
+@pytest.mark.parametrize("nheads,sizes", [(1, (3072,)), (1, (16,)), (8, (256,)), (8, (48,)), (2, (16, 24, 256, 384)),
+                                          (8, (128, 192, 2048, 3072))])
+def test_marks_follow_the_counts_of_many_waves(heap, nheads, sizes):
+    # the heap is filled until hamalloc returns NULL, then a share of the blocks
+    # is freed again and again while other waves allocate: many slabs pass the
+    # threshold in both directions, between them in one kernel (loops on a heap
+    # kept near full), and every full slab is marked at the end of each step
+    print(f"[gpu] full marks nheads={nheads} sizes={sizes}", flush=True)
+    heap(H.HallocOpts(memory=40 << 20, sb_sz_sh=21, nheads=nheads))
+    rng = np.random.default_rng(len(sizes) + nheads)
+    n = int(1.3 * H.Halloc.geometry()["arena_bytes"] / np.mean(sizes))
+    live = np.zeros(0, np.uint64)
+    seen = 0
+    for keep in (0.9, 0.8, 0.95, 0.5, 0.85, 0.0):
+        p = H.Halloc.malloc_sizes(rng.choice(sizes, max(n - live.size, 64)).astype(np.uint32), 256)
+        live = np.concatenate([live, p[p != 0]])
+        rng.shuffle(live)
+        full, bad = unmarked_full_slabs()
+        assert not bad
+        seen += full
+        k = int(keep * live.size)
+        H.Halloc.free_ptrs(live[k:])
+        live = live[:k]
+        assert not unmarked_full_slabs()[1]
+        for sz in sizes:
+            r = run("priv-throughput", 4000, 128, sz, ntries=3, memory=40 << 20)
+            assert r["mallocs"] == r["frees"]
+            assert not unmarked_full_slabs()[1]
+    assert seen > 0 and live.size == 0
+    assert H.Halloc.free_bytes() == H.Halloc.geometry()["arena_bytes"]
+
+
 @pytest.mark.parametrize("length", [1, 15, 16, 17, 33, 64])
 @pytest.mark.parametrize("nreq", [1, 3, 64, 256, 700])
 def test_pages_drained_together(heap, nreq, length):

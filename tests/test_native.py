@@ -1,6 +1,7 @@
 """CPU checks of the arithmetic shared with the device code: the wave-run layout and division-free
-remainders (halloc_amd/csrc/ha_bits.h) against brute force, and the graph workload's Poisson table
-(halloc_amd/csrc/ha_workload.h) against scipy."""
+remainders (halloc_amd/csrc/ha_bits.h) against brute force, the graph workload's Poisson table
+(halloc_amd/csrc/ha_workload.h) against scipy, and the slabs' full marks (halloc_amd/csrc/ha_mark.h)
+in every interleaving of a few groups."""
 import os
 import subprocess
 
@@ -40,6 +41,15 @@ def test_graph_item_sequence(tmp_path):
     exe = tmp_path / "graph_seq_check"
     subprocess.run(["g++", "-O2", "-std=c++17", "-o", str(exe),
                     os.path.join(HERE, "native", "graph_seq_check.cpp")], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert r.stdout.strip() == "ok"
+
+
+def test_full_mark_interleavings(tmp_path):
+    exe = tmp_path / "full_mark_check"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-o", str(exe),
+                    os.path.join(HERE, "native", "full_mark_check.cpp")], check=True)
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout + r.stderr
     assert r.stdout.strip() == "ok"
