@@ -182,8 +182,12 @@ struct DBuf {
       pool().trim();
       e = hipMalloc(&p, cap);
     }
-    if (e != hipSuccess) p = nullptr;
-    else ++t_held;
+    if (e != hipSuccess) {
+      (void)hipGetLastError();  // reported here, not by a later call
+      p = nullptr;
+    } else {
+      ++t_held;
+    }
     return e;
   }
 };
@@ -200,20 +204,21 @@ struct Stream {
   }
 };
 
-hipError_t event_get(hipEvent_t* e) {
-  int dev = 0;
-  if (hipError_t r = hipGetDevice(&dev)) return r;
-  return take(pool().events, dev, e) ? hipSuccess : hipEventCreate(e);
-}
-void event_put(hipEvent_t e) {
-  if (!keep(pool().events, Pool::MAX_EVENTS, e)) (void)hipEventDestroy(e);
-}
-
-struct Events {
-  std::vector<hipEvent_t> e;
-  ~Events() {
-    for (hipEvent_t x : e) event_put(x);
+// Event that gives itself back, on every way out of a driver.
+struct Event {
+  hipEvent_t e = nullptr;
+  Event() = default;
+  Event(const Event&) = delete;
+  Event(Event&& o) noexcept : e(o.e) { o.e = nullptr; }
+  ~Event() {
+    if (e && !keep(pool().events, Pool::MAX_EVENTS, e)) (void)hipEventDestroy(e);
   }
+  hipError_t create() {
+    int dev = 0;
+    if (hipError_t r = hipGetDevice(&dev)) return r;
+    return take(pool().events, dev, &e) ? hipSuccess : hipEventCreate(&e);
+  }
+  operator hipEvent_t() const { return e; }
 };
 
 // ------------------------------------------------------------------ replay
@@ -2042,12 +2047,8 @@ int ha_run_plain(int nthreads, int bs, int size, int iters, int warmup, int laun
   HH(s.create());
   // ev[0], ev[1]: the timed region; ev[2 + 2l], ev[3 + 2l]: launch l of the
   // per-launch pass
-  Events ev;
-  for (int i = 0; i < 2 + (ms ? 2 * launches : 0); ++i) {
-    hipEvent_t e;
-    HH(event_get(&e));
-    ev.e.push_back(e);
-  }
+  std::vector<Event> ev(2 + (ms ? 2 * (size_t)launches : 0));
+  for (Event& e : ev) HH(e.create());
   const int grid = (nthreads + bs - 1) / bs;
   unsigned long long* c = (unsigned long long*)dc.p;
   for (int w = 0; w < warmup; ++w) plain_k<<<grid, bs, 0, s.s>>>(nthreads, size, iters, c, c + 1);
@@ -2059,24 +2060,24 @@ int ha_run_plain(int nthreads, int bs, int size, int iters, int warmup, int laun
   // launches runs: no host synchronization and no event between them (an
   // event pair around every launch lengthened each step by about 6 us)
   const auto w0 = std::chrono::steady_clock::now();
-  HH(hipEventRecord(ev.e[0], s.s));
+  HH(hipEventRecord(ev[0], s.s));
   for (int l = 0; l < launches; ++l) plain_k<<<grid, bs, 0, s.s>>>(nthreads, size, iters, c, c + 1);
-  HH(hipEventRecord(ev.e[1], s.s));
+  HH(hipEventRecord(ev[1], s.s));
   HH(hipStreamSynchronize(s.s));
   const auto w1 = std::chrono::steady_clock::now();
   HH(hipGetLastError());
   float total = 0;
-  HH(hipEventElapsedTime(&total, ev.e[0], ev.e[1]));
+  HH(hipEventElapsedTime(&total, ev[0], ev[1]));
   if (ms) {
     // the per-launch pass, after the timed region
     for (int l = 0; l < launches; ++l) {
-      HH(hipEventRecord(ev.e[2 + 2 * l], s.s));
+      HH(hipEventRecord(ev[2 + 2 * l], s.s));
       plain_k<<<grid, bs, 0, s.s>>>(nthreads, size, iters, c, c + 1);
-      HH(hipEventRecord(ev.e[3 + 2 * l], s.s));
+      HH(hipEventRecord(ev[3 + 2 * l], s.s));
     }
     HH(hipStreamSynchronize(s.s));
     HH(hipGetLastError());
-    for (int l = 0; l < launches; ++l) HH(hipEventElapsedTime(&ms[l], ev.e[2 + 2 * l], ev.e[3 + 2 * l]));
+    for (int l = 0; l < launches; ++l) HH(hipEventElapsedTime(&ms[l], ev[2 + 2 * l], ev[3 + 2 * l]));
   }
   unsigned long long h[2];
   HH(hipMemcpy(h, dc.p, 16, hipMemcpyDeviceToHost));
@@ -2115,9 +2116,9 @@ int ha_run_corr_test0(int nthreads, int nmallocs, int bs, ha_corr0_result* r) {
   HH(hipMemset(dp.p, 0, n * 8));
   HH(hipMemset(dc.p, 0, 16));
   unsigned long long* cnt = (unsigned long long*)dc.p;
-  hipEvent_t e1, e2;
-  HH(event_get(&e1));
-  HH(event_get(&e2));
+  Event e1, e2;
+  HH(e1.create());
+  HH(e2.create());
   t0_malloc_k<<<nthreads / bs, bs>>>((void**)dp.p, nmallocs, cnt);
   HH(hipGetLastError());
   const unsigned g = (unsigned)((n + 255) / 256);
@@ -2145,8 +2146,6 @@ int ha_run_corr_test0(int nthreads, int nmallocs, int bs, ha_corr0_result* r) {
   r->blocks = n;
   r->nulls = h[0];
   r->bad_contents = h[1];
-  event_put(e1);
-  event_put(e2);
   return HA_OK;
 }
 
@@ -2189,9 +2188,9 @@ int ha_run_touch(int n, int words, int iters, int reps, double* ms, uint64_t* su
   HH(hipMemset(dn.p, 0, 8));
   Stream s;
   HH(s.create());
-  hipEvent_t e0, e1;
-  HH(event_get(&e0));
-  HH(event_get(&e1));
+  Event e0, e1;
+  HH(e0.create());
+  HH(e1.create());
   u64** ptrs = (u64**)dp.p;
   u64* sink = (u64*)ds.p;
   touch_alloc_k<<<grid, bs, 0, s.s>>>(ptrs, n, words, (unsigned long long*)dn.p);
@@ -2219,8 +2218,6 @@ int ha_run_touch(int n, int words, int iters, int reps, double* ms, uint64_t* su
   HH(hipGetLastError());
   HH(hipMemcpyAsync(nulls, dn.p, 8, hipMemcpyDeviceToHost, s.s));
   HH(hipStreamSynchronize(s.s));
-  event_put(e0);
-  event_put(e1);
   return HA_OK;
 }
 
@@ -2232,9 +2229,9 @@ int ha_probe_atomics(double* out) {
   HH(buf.alloc(BYTES));
   HH(sink.alloc((size_t)NT * 8));
   HH(hipMemset(buf.p, 0, BYTES));
-  hipEvent_t e0, e1;
-  HH(event_get(&e0));
-  HH(event_get(&e1));
+  Event e0, e1;
+  HH(e0.create());
+  HH(e1.create());
   const u64 mask = BYTES / 8 - 1;
   for (int shape = 0; shape < 3; ++shape) {
     const int iters = shape == 2 ? 1 : 16;
@@ -2251,8 +2248,6 @@ int ha_probe_atomics(double* out) {
     out[shape] = (double)NT * iters / (best * 1e-3);
   }
   HH(hipGetLastError());
-  event_put(e0);
-  event_put(e1);
   return HA_OK;
 }
 
@@ -2267,9 +2262,9 @@ int ha_probe_chain(const int* rounds, int n, int nthreads, double* ms) {
   HH(buf.alloc(BYTES));
   HH(sink.alloc((size_t)nthreads / 64 * 8));
   HH(hipMemset(buf.p, 0, BYTES));
-  hipEvent_t e0, e1;
-  HH(event_get(&e0));
-  HH(event_get(&e1));
+  Event e0, e1;
+  HH(e0.create());
+  HH(e1.create());
   for (int i = 0; i < n; ++i) {
     float best = 1e30f;
     for (int rep = 0; rep < 5; ++rep) {
@@ -2284,8 +2279,6 @@ int ha_probe_chain(const int* rounds, int n, int nthreads, double* ms) {
     ms[i] = best;
   }
   HH(hipGetLastError());
-  event_put(e0);
-  event_put(e1);
   return HA_OK;
 }
 
@@ -2324,9 +2317,9 @@ int ha_run_test(const ha_test_opts* a, ha_test_result* r) {
   const bool stamped = a->test == 0 || a->test == 1;
   Stream s;
   HH(s.create());
-  hipEvent_t e0, e1;
-  HH(event_get(&e0));
-  HH(event_get(&e1));
+  Event e0, e1;
+  HH(e0.create());
+  HH(e1.create());
   // acc: kernel time from events; the wall-clock time around launch and
   // synchronization (what the reference's tests report, omp_get_wtime) goes
   // to the matching *_wall_ms field
@@ -2464,8 +2457,6 @@ int ha_run_test(const ha_test_opts* a, ha_test_result* r) {
     r->lat_min[k] = l[4 * k] ? (double)l[4 * k + 2] : 0.0;
     r->lat_max[k] = (double)l[4 * k + 3];
   }
-  event_put(e0);
-  event_put(e1);
   return HA_OK;
 }
 
@@ -2480,8 +2471,8 @@ int ha_run_sample(const ha_sample_args* a, ha_sample_result* r) {
   const u32 n = (u32)a->n;
   Stream s;
   HH(s.create());
-  hipEvent_t e[5];  // alloc, work, free: e0-e1, e1-e2, e3-e4
-  for (auto& x : e) HH(event_get(&x));
+  Event e[5];  // alloc, work, free: e0-e1, e1-e2, e3-e4
+  for (Event& x : e) HH(x.create());
   DBuf dst;
   HH(dst.alloc(4 * 8));
   HH(hipMemset(dst.p, 0, 4 * 8));
@@ -2567,7 +2558,6 @@ int ha_run_sample(const ha_sample_args* a, ha_sample_result* r) {
   r->alloc_ms = t[0];
   r->work_ms = t[1];
   r->free_ms = t[2];
-  for (auto& x : e) event_put(x);
   return HA_OK;
 }
 
@@ -2586,9 +2576,9 @@ int ha_probe_copy(uint64_t bytes, int reps, double* gbps) {
   const int grid = ncu * 8;
   Stream s;
   HH(s.create());
-  hipEvent_t e0, e1;
-  HH(event_get(&e0));
-  HH(event_get(&e1));
+  Event e0, e1;
+  HH(e0.create());
+  HH(e1.create());
   float best = 1e30f;
   for (int r = 0; r < reps; ++r) {
     HH(hipEventRecord(e0, s.s));
@@ -2600,8 +2590,6 @@ int ha_probe_copy(uint64_t bytes, int reps, double* gbps) {
     best = t < best ? t : best;
   }
   HH(hipGetLastError());
-  event_put(e0);
-  event_put(e1);
   *gbps = 2.0 * (double)bytes / (best * 1e-3) / 1e9;
   return HA_OK;
 }
@@ -2615,29 +2603,28 @@ int ha_run_lists(const uint32_t* sizes, int n, int per, const uint32_t* order, i
   // slots takes 210 us with the host's loops and 215 with the kernels, over
   // 128 Ki 280 and 255 (without an order 154 and 152, 166 and 163)
   const bool scan = total >= LIST_SCAN_MIN;
-  if (order && !scan) {
+  auto permutation = [&] {
     std::vector<uint8_t> seen(total, 0);
     for (size_t k = 0; k < total; ++k) {
-      if (order[k] >= total || seen[order[k]]) return hfail(HA_E_INVALID, "order is not a permutation");
+      if (order[k] >= total || seen[order[k]]) return false;
       seen[order[k]] = 1;
     }
-  }
+    return true;
+  };
+  if (order && !scan && !permutation()) return hfail(HA_E_INVALID, "order is not a permutation");
   DBuf ds, dp, dord, dc;
-  HH(ds.alloc(total * 4));
-  HH(dp.alloc(total * 8));
-  HH(dc.alloc(32));  // NULLs, bad stamps, then the scan's requests and lost places
+  hipError_t mem = ds.alloc(total * 4);
+  if (!mem) mem = dp.alloc(total * 8);
+  if (!mem) mem = dc.alloc(32);  // NULLs, bad stamps, then the scan's requests and lost places
+  if (!mem && order) mem = dord.alloc(total * 4);
+  // no memory for the device's check: a bad order is still refused as one
+  if (mem && order && scan && !permutation()) return hfail(HA_E_INVALID, "order is not a permutation");
+  if (mem) return hfail(HA_E_HIP, std::string("device buffers of the lists: ") + hipGetErrorString(mem));
   HH(hipMemcpy(ds.p, sizes, total * 4, hipMemcpyHostToDevice));
-  if (order) {
-    HH(dord.alloc(total * 4));
-    HH(hipMemcpy(dord.p, order, total * 4, hipMemcpyHostToDevice));
-  }
+  if (order) HH(hipMemcpy(dord.p, order, total * 4, hipMemcpyHostToDevice));
   HH(hipMemset(dc.p, 0, 32));
   Stream s;
   HH(s.create());
-  hipEvent_t e0, e1, e2;
-  HH(event_get(&e0));
-  HH(event_get(&e1));
-  HH(event_get(&e2));
   unsigned long long* c = (unsigned long long*)dc.p;
   const int grid = (n + bs - 1) / bs;
   unsigned long long h[4];
@@ -2651,6 +2638,10 @@ int ha_run_lists(const uint32_t* sizes, int n, int per, const uint32_t* order, i
       if (h[3]) return hfail(HA_E_INVALID, "order is not a permutation");
     }
   }
+  Event e0, e1, e2;
+  HH(e0.create());
+  HH(e1.create());
+  HH(e2.create());
   HH(hipStreamSynchronize(s.s));
   const auto w0 = std::chrono::steady_clock::now();
   HH(hipEventRecord(e0, s.s));
@@ -2670,9 +2661,6 @@ int ha_run_lists(const uint32_t* sizes, int n, int per, const uint32_t* order, i
   HH(hipEventElapsedTime(&tm, e0, e1));
   HH(hipEventElapsedTime(&tf, e1, e2));
   HH(hipMemcpy(h, dc.p, 32, hipMemcpyDeviceToHost));
-  event_put(e0);
-  event_put(e1);
-  event_put(e2);
   res->nulls = h[0];
   res->errors = h[1];
   res->malloc_ms = tm;
@@ -2700,9 +2688,9 @@ int ha_run_phase(const ha_phase_args* a, ha_phase_result* res, double* trace, in
   HH(hipMemset(dc.p, 0, 8 * 8));
   Stream s;
   HH(s.create());
-  hipEvent_t e0, e1;
-  HH(event_get(&e0));
-  HH(event_get(&e1));
+  Event e0, e1;
+  HH(e0.create());
+  HH(e1.create());
   unsigned long long* c = (unsigned long long*)dc.p;
   const int grid = (n + a->bs - 1) / a->bs;
   const double heap = (double)P.arena_bytes;
@@ -2756,8 +2744,6 @@ int ha_run_phase(const ha_phase_args* a, ha_phase_result* res, double* trace, in
   wall += std::chrono::duration<double, std::milli>(w1 - w0).count();
   HH(hipGetLastError());
   HH(hipMemcpy(h, dc.p, sizeof h, hipMemcpyDeviceToHost));
-  event_put(e0);
-  event_put(e1);
   res->mallocs = h[0];
   res->frees = h[1];
   res->nulls = h[2];
@@ -2821,9 +2807,9 @@ int ha_run_graphs(const ha_graph_args* a, const uint32_t* nnodes, ha_graph_resul
   HH(hipMemset(dstats.p, 0, 16));
   Stream s;
   HH(s.create());
-  hipEvent_t e0, e1;
-  HH(event_get(&e0));
-  HH(event_get(&e1));
+  Event e0, e1;
+  HH(e0.create());
+  HH(e1.create());
   unsigned long long* st = (unsigned long long*)dstats.p;
   std::memset(res, 0, sizeof *res);
   res->nodes = total;
@@ -2955,8 +2941,6 @@ int ha_run_graphs(const ha_graph_args* a, const uint32_t* nnodes, ha_graph_resul
   HH(hipMemcpy(h, dstats.p, 16, hipMemcpyDeviceToHost));
   (void)hipGraphExecDestroy(exec);
   (void)hipGraphDestroy(graph);
-  event_put(e0);
-  event_put(e1);
   res->nulls = h[0];
   res->errors = h[1];
   res->plain_ms = a->run_plain ? best_plain : 0;
@@ -3038,9 +3022,9 @@ int ha_run_serve(const ha_serve_io* io, ha_serve_result* res) {
   a.lat_cap = (u32)io->lat_cap;
   Stream s;
   HH(s.create());
-  hipEvent_t e0, e1;
-  HH(event_get(&e0));
-  HH(event_get(&e1));
+  Event e0, e1;
+  HH(e0.create());
+  HH(e1.create());
   HH(hipEventRecord(e0, s.s));
   srv_start_k<<<1, 1, 0, s.s>>>(a.st);
   srv_loop_k<<<io->slots / 256, 256, 0, s.s>>>(a);
@@ -3049,8 +3033,6 @@ int ha_run_serve(const ha_serve_io* io, ha_serve_result* res) {
   HH(hipGetLastError());
   float t = 0;
   HH(hipEventElapsedTime(&t, e0, e1));
-  event_put(e0);
-  event_put(e1);
   SrvState fin;
   HH(hipMemcpy(&fin, dst.p, sizeof fin, hipMemcpyDeviceToHost));
   HH(hipMemcpy(io->checksum, dcs.p, n * 4, hipMemcpyDeviceToHost));
