@@ -1605,11 +1605,14 @@ static Params g_host;          // host copy of ha_p
 static void* g_meta = nullptr;  // one allocation for all metadata
 
 static thread_local std::string g_err;
+static thread_local unsigned long long g_fails = 0;  // errors reported in this thread
 
 int fail(int code, const std::string& msg) {
   g_err = msg;
+  ++g_fails;
   return code;
 }
+unsigned long long fail_count() { return g_fails; }
 #define HA_HIP(call)                                                                              \
   do {                                                                                            \
     hipError_t e_ = (call);                                                                       \

@@ -31,6 +31,7 @@ __device__ void hafree_batch(void* const* ptrs, int cnt);
 namespace ha {
 const Params& host_params();
 int fail(int code, const std::string& msg);
+unsigned long long fail_count();
 void on_release(void (*f)());
 }
 
@@ -41,14 +42,7 @@ using ha::u64;
 
 namespace {
 
-// this thread's driver call: whether it failed, and the buffers it holds
-thread_local bool t_failed = false;
-thread_local int t_held = 0;
-
-int hfail(int code, const std::string& m) {
-  t_failed = true;
-  return ha::fail(code, m);
-}
+int hfail(int code, const std::string& m) { return ha::fail(code, m); }
 
 #define HH(call)                                                                                 \
   do {                                                                                           \
@@ -105,8 +99,14 @@ Pool& pool() {
   }();
   return *p;
 }
-// the driver call that gives back succeeded: no error, no exception under way
-bool finished() { return !t_failed && std::uncaught_exceptions() == 0; }
+// What the pool's objects keep of the call that holds them.  good(): nothing
+// failed in this thread since the object was made (every error, the
+// allocator's own too, is reported through ha::fail) and no exception is under
+// way, so the driver call that lets go of it is returning HA_OK.
+struct Held {
+  const unsigned long long fails = ha::fail_count();
+  bool good() const { return ha::fail_count() == fails && std::uncaught_exceptions() == 0; }
+};
 
 template <class T>
 bool take(std::vector<std::pair<int, T>>& v, int dev, T* out) {
@@ -120,9 +120,9 @@ bool take(std::vector<std::pair<int, T>>& v, int dev, T* out) {
   return false;
 }
 template <class T>
-bool keep(std::vector<std::pair<int, T>>& v, size_t most, T x) {
+bool keep(const Held& held, std::vector<std::pair<int, T>>& v, size_t most, T x) {
   int dev = 0;
-  if (!finished() || hipGetDevice(&dev) != hipSuccess) return false;
+  if (!held.good() || hipGetDevice(&dev) != hipSuccess) return false;
   std::lock_guard<std::mutex> g(pool().mu);
   if (v.size() >= most) return false;
   v.emplace_back(dev, x);
@@ -134,10 +134,10 @@ struct DBuf {
   void* p = nullptr;
   size_t cap = 0;
   int dev = 0;
+  Held held;
   ~DBuf() {
     if (!p) return;
-    --t_held;
-    if (!finished() || cap > Pool::MAX_BYTES) {
+    if (!held.good() || cap > Pool::MAX_BYTES) {
       (void)hipFree(p);
       return;
     }
@@ -154,7 +154,6 @@ struct DBuf {
   // at least n bytes: the smallest buffer kept for this device that holds n
   // and is at most twice as large, or a new one
   hipError_t alloc(size_t n) {
-    if (t_held == 0) t_failed = false;  // a new call's first buffer
     if (hipError_t e = hipGetDevice(&dev)) return e;
     if (n > Pool::MAX_BYTES) {
       cap = n;
@@ -172,7 +171,6 @@ struct DBuf {
         cap = q.bufs[best].n;
         q.bytes -= cap;
         q.bufs.erase(q.bufs.begin() + (std::ptrdiff_t)best);
-        ++t_held;
         return hipSuccess;
       }
     }
@@ -185,8 +183,6 @@ struct DBuf {
     if (e != hipSuccess) {
       (void)hipGetLastError();  // reported here, not by a later call
       p = nullptr;
-    } else {
-      ++t_held;
     }
     return e;
   }
@@ -194,8 +190,9 @@ struct DBuf {
 
 struct Stream {
   hipStream_t s = nullptr;
+  Held held;
   ~Stream() {
-    if (s && !keep(pool().streams, Pool::MAX_STREAMS, s)) (void)hipStreamDestroy(s);
+    if (s && !keep(held, pool().streams, Pool::MAX_STREAMS, s)) (void)hipStreamDestroy(s);
   }
   hipError_t create() {
     int dev = 0;
@@ -207,11 +204,12 @@ struct Stream {
 // Event that gives itself back, on every way out of a driver.
 struct Event {
   hipEvent_t e = nullptr;
+  Held held;
   Event() = default;
   Event(const Event&) = delete;
-  Event(Event&& o) noexcept : e(o.e) { o.e = nullptr; }
+  Event(Event&& o) noexcept : e(o.e), held(o.held) { o.e = nullptr; }
   ~Event() {
-    if (e && !keep(pool().events, Pool::MAX_EVENTS, e)) (void)hipEventDestroy(e);
+    if (e && !keep(held, pool().events, Pool::MAX_EVENTS, e)) (void)hipEventDestroy(e);
   }
   hipError_t create() {
     int dev = 0;
@@ -2396,12 +2394,8 @@ int ha_run_test(const ha_test_opts* a, ha_test_result* r) {
                            t % 2 ? r->free_ms : r->malloc_ms))
           return rc;
         if (a->test == 8 && a->extfrag) {
-          int rc = ha_extfrag_c(0, &a->extfrag[2 * t]);
-          if (!rc) rc = ha_extfrag_c(1, &a->extfrag[2 * t + 1]);
-          if (rc) {
-            t_failed = true;
-            return rc;
-          }
+          if (int rc = ha_extfrag_c(0, &a->extfrag[2 * t])) return rc;
+          if (int rc = ha_extfrag_c(1, &a->extfrag[2 * t + 1])) return rc;
         }
         if (int rc = check_nz(true, t)) return rc;
         break;
