@@ -32,7 +32,8 @@ EXPORTS = ("ha_default_opts", "ha_init_c", "ha_shutdown_c", "ha_extfrag_c", "ha_
            "ha_run_plain", "ha_malloc_sizes", "ha_free_ptrs", "ha_read_words", "ha_probe_atomics",
            "ha_run_lists", "ha_run_phase", "ha_replay_batch", "ha_run_graphs", "ha_run_serve",
            "ha_probe_copy", "ha_run_test", "ha_run_sample", "ha_run_corr_test0", "ha_probe_chain",
-           "ha_free_bytes_noalloc_c", "ha_run_touch", "ha_full_marks")
+           "ha_free_bytes_noalloc_c", "ha_run_touch", "ha_full_marks",
+           "ha_release_buffers")
 
 
 class HallocError(RuntimeError):
@@ -197,6 +198,7 @@ def lib() -> ctypes.CDLL:
         "ha_dump_words": (ctypes.c_int64, []),
         "ha_dump": (i32, [vp, ctypes.c_int64]),
         "ha_full_marks": (i32, [vp, ctypes.c_int64]),
+        "ha_release_buffers": (i32, []),
         "ha_run_plain": (i32, [i32, i32, i32, i32, i32, i32, vp, P(_PlainResult)]),
         "ha_malloc_sizes": (i32, [vp, i32, i32, vp]),
         "ha_run_corr_test0": (i32, [i32, i32, i32, P(_Corr0Result)]),
@@ -240,6 +242,11 @@ class Halloc:
     @staticmethod
     def shutdown() -> None:
         _check(lib().ha_shutdown_c())
+
+    @staticmethod
+    def release_buffers() -> None:
+        """Gives back the device memory, streams and events the drivers keep between calls."""
+        _check(lib().ha_release_buffers())
 
     @staticmethod
     def extfrag(ideal: bool) -> float:

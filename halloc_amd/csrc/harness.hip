@@ -59,15 +59,17 @@ int hfail(int code, const std::string& m) { return ha::fail(code, m); }
 // A call that failed gives nothing back: it may have left work behind, and
 // hipFree and hipStreamDestroy wait for it.  A call that returns HA_OK has
 // waited for its work.  Contents are undefined, as from hipMalloc.  Bounded (the
-// oldest buffers go first), emptied by ha_init, ha_shutdown and when an
-// allocation fails, and locked, so drivers may run in several threads.
+// oldest buffers go first) to what the largest of these workloads holds at
+// once, since it is memory that a caller's own hipMalloc cannot have; emptied
+// by ha_init, ha_shutdown, ha_release_buffers and when an allocation here
+// fails; and locked, so drivers may run in several threads.
 struct Pool {
   struct Buf {
     int dev;
     void* p;
     size_t n;
   };
-  static constexpr size_t MAX_BYTES = 512ull << 20, MAX_BUFS = 32, MAX_STREAMS = 8, MAX_EVENTS = 64;
+  static constexpr size_t MAX_BYTES = 256ull << 20, MAX_BUFS = 32, MAX_STREAMS = 8, MAX_EVENTS = 64;
   std::mutex mu;
   std::vector<Buf> bufs;  // oldest first
   std::vector<std::pair<int, hipStream_t>> streams;
@@ -2020,6 +2022,11 @@ int ha_dump(uint64_t* out, int64_t nwords) {
   dump_k<<<1024, 256>>>((u64*)d.p, total);
   HH(hipGetLastError());
   HH(hipMemcpy(out, d.p, total * 8, hipMemcpyDeviceToHost));
+  return HA_OK;
+}
+
+int ha_release_buffers(void) {
+  pool().trim();
   return HA_OK;
 }
 

@@ -68,6 +68,11 @@ void ha_default_opts(ha_opts_c *o);
 int ha_init_c(const ha_opts_c *o);
 /* Replaces ha_shutdown (src/halloc.cu:426-428); frees the pool. */
 int ha_shutdown_c(void);
+/* The workload drivers below keep device buffers (256 MiB at most), streams and
+   events for their next calls.  This gives them back, as ha_init_c and
+   ha_shutdown_c do: for a program that needs the memory itself.  The heap and
+   calls under way in other threads are not touched. */
+int ha_release_buffers(void);
 /* Replaces ha_extfrag (src/statistics.cuh:50-69).  Writes the value to *out. */
 int ha_extfrag_c(int ideal, double *out);
 /* Free bytes of the slab heap, the counterpart of find_free_mem_k

@@ -167,3 +167,23 @@ for pooled in (False, True):
         left = [live(i) for i in (STREAMS, EVENTS, BUFFERS, WRONG)]
         assert left == [0] * 4, (k, left)
 """ % (DRIVERS[name], name in ("points", "strings", "arrays")))
+
+
+def test_kept_buffers_are_bounded_and_given_back(fake):
+    # what finished calls leave for later ones stays within its bound, and one
+    # call gives it back while the heap lives
+    run(fake, """
+H.Halloc.init(OPTS)
+base, heap = live(BUFFERS), live(USED)
+for n in (1 << 10, 1 << 20, 5 << 20, 1 << 20, 9 << 20, 7 << 20, 3):
+    H.Halloc.run_lists(np.full((1, n), 16, np.uint32))
+    assert live(USED) - heap <= 256 << 20, (n, live(USED) - heap)
+    assert live(BUFFERS) - base <= 32
+assert live(USED) > heap and live(STREAMS) and live(EVENTS)
+H.Halloc.release_buffers()
+assert [live(i) for i in (STREAMS, EVENTS, BUFFERS, WRONG)] == [0, 0, base, 0] and live(USED) == heap
+assert H.Halloc.run_lists(np.full((1, 100), 16, np.uint32))["requests"] == 100
+H.Halloc.release_buffers()
+H.Halloc.release_buffers()
+assert live(USED) == heap
+""")
