@@ -33,7 +33,7 @@ EXPORTS = ("ha_default_opts", "ha_init_c", "ha_shutdown_c", "ha_extfrag_c", "ha_
            "ha_run_lists", "ha_run_phase", "ha_replay_batch", "ha_run_graphs", "ha_run_serve",
            "ha_probe_copy", "ha_run_test", "ha_run_sample", "ha_run_corr_test0", "ha_probe_chain",
            "ha_free_bytes_noalloc_c", "ha_run_touch", "ha_full_marks",
-           "ha_release_buffers")
+           "ha_release_buffers", "ha_check_pages")
 
 
 class HallocError(RuntimeError):
@@ -213,6 +213,7 @@ def lib() -> ctypes.CDLL:
         "ha_replay_batch": (i32, [vp, i32, i32, vp, vp]),
         "ha_run_graphs": (i32, [P(_GraphArgs), vp, P(_GraphResult)]),
         "ha_run_serve": (i32, [P(_ServeIO), P(_ServeResult)]),
+        "ha_check_pages": (i32, [vp] * 8),
         "ha_probe_copy": (i32, [u64, i32, P(ctypes.c_double)]),
         "ha_run_test": (i32, [P(_TestOpts), P(_TestResult)]),
         "ha_run_sample": (i32, [P(_SampleArgs), P(_SampleResult)]),
@@ -466,6 +467,19 @@ class Halloc:
         _check(lib().ha_run_graphs(ctypes.byref(a), nn.ctypes.data, ctypes.byref(r)))
         return {"nodes": int(r.nodes), "nulls": int(r.nulls), "errors": int(r.errors),
                 "plain_ms": r.plain_ms, "batch_ms": r.batch_ms, "plain_launches": int(r.plain_launches)}
+
+    @staticmethod
+    def check_pages(pages, tag, drain, tok, drains, checksum, bad, bad_first):
+        """The serving loop's page check on prepared pages, one step of one wave
+        (64 lanes).  Returns the updated (checksum, bad, bad_first)."""
+        pg = np.ascontiguousarray(pages, dtype=np.uint32)
+        ins = [np.ascontiguousarray(x, dtype=np.uint32) for x in (tag, drain, tok, drains)]
+        cs, nb = np.array(checksum, dtype=np.uint32), np.array(bad, dtype=np.uint32)
+        bf = np.array(bad_first, dtype=np.uint64)
+        if pg.shape != (64, 16, 4) or any(x.shape != (64,) for x in (*ins, cs, nb, bf)):
+            raise ValueError("pages must be (64, 16, 4), the other arrays (64,)")
+        _check(lib().ha_check_pages(*(x.ctypes.data for x in (pg, *ins, cs, nb, bf))))
+        return cs, nb, bf
 
     @staticmethod
     def run_serve(arrival_ns, length, tag, slots=65536, watermark=64 << 20, sample_every=8, lat_cap=1 << 22):

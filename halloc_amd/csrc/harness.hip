@@ -1211,14 +1211,33 @@ __device__ __forceinline__ u32 wave_sum(u32 v) {
   return v;
 }
 
-// One pass of the shared page check: lane 16 g + j holds token j of the page
-// of the g-th draining lane in the pass (owner[g]; 64: none).  Every lane of
-// the wave takes part.
+// The check of the pages that a wave's lanes drain in one step.  Up to
+// DRAIN_SHARED lanes share it with the whole wave: one token per lane, four
+// pages at a time, one coalesced load each time, the first of them under way
+// while other lanes allocate.  In most steps of a mixed load a few of the 64
+// lanes drain, and lanes that checked their own pages made the wave run 16
+// hashes one after another: 20 000 requests of mixed lengths take 7.2 ms, and
+// 8.4 if every lane checks its own page.  A pass is about 0.7 us of cross-lane
+// work, though, so with more lanes each checks its own: 1024 waves of k
+// sequences of 256 tokens in step take, shared | own, 419 | 412 us at k = 4,
+// 434 | 422 at 8, 460 | 430 at 16, 483 | 437 at 24, 784 | 642 at 64.  Sequences
+// of one length that arrive together drain all at once: 65 536 of 64 and of 256
+// tokens 180 and 775 us with every page shared, 155 and 658 with this rule.
+// Heap pages are global memory, and the loads say so: a generic load counts as
+// an LDS access too, and the next pass's permutes would wait for it.
+constexpr u32 DRAIN_SHARED = 8;
+constexpr u32 OWN_TOKENS = 4;  // loads in flight of a lane's own check
+typedef u32 u32x4 __attribute__((ext_vector_type(4)));
+typedef const __attribute__((address_space(1))) u32x4* gpage;
+
+// One pass of the shared check: lane 16 g + j holds token j of the page of the
+// g-th draining lane in the pass (owner[g]; 64: none).  Every lane of the wave
+// takes part.
 struct DrainPass {
   u32 owner[4];
   u32 tag, t, any;
   bool has;
-  uint4 v;
+  u32x4 v;
 };
 __device__ __forceinline__ u32 lane_of(u32 v, u32 src) {
   return (u32)__builtin_amdgcn_ds_bpermute((int)(src << 2), (int)v);
@@ -1229,7 +1248,7 @@ __device__ __forceinline__ DrainPass drain_load(u64& rem, u32 me, const uint4* p
   d.any = rem != 0;
   d.has = false;
   d.tag = d.t = 0;
-  d.v = make_uint4(0u, 0u, 0u, 0u);
+  d.v = u32x4{0u, 0u, 0u, 0u};
   if (!d.any) return d;
   u32 src = 64;
 #pragma unroll
@@ -1244,7 +1263,7 @@ __device__ __forceinline__ DrainPass drain_load(u64& rem, u32 me, const uint4* p
   d.t = lane_of(drain, from) * SRV_TOK_PER_PAGE + (me & 15u);
   const u32 n = lane_of(tok, from);
   d.has = src < 64 && d.t < n;
-  if (d.has) d.v = ((const uint4*)((u64)hi << 32 | lo))[me & 15u];
+  if (d.has) d.v = ((gpage)((u64)hi << 32 | lo))[me & 15u];
   return d;
 }
 // adds the pass's hashes and damaged tokens to their owners
@@ -1274,6 +1293,70 @@ __device__ __forceinline__ void drain_check(const DrainPass& d, u32 me, u32& cs,
       }
     }
   }
+}
+
+// A lane's check of its own page.
+__device__ __forceinline__ void drain_own(const uint4* pg, u32 tag, u32 drain, u32 tok, u32& cs, u32& nbad,
+                                          u64& first_bad) {
+  const u32 t0 = drain * SRV_TOK_PER_PAGE;
+  const u32 n = tok - t0 < SRV_TOK_PER_PAGE ? tok - t0 : SRV_TOK_PER_PAGE;
+#pragma nounroll
+  for (u32 j0 = 0; j0 < n; j0 += OWN_TOKENS) {
+    u32x4 v[OWN_TOKENS];
+#pragma unroll
+    for (u32 j = 0; j < OWN_TOKENS; ++j)
+      if (j0 + j < n) v[j] = ((gpage)(u64)pg)[j0 + j];
+#pragma unroll
+    for (u32 j = 0; j < OWN_TOKENS; ++j) {
+      if (j0 + j >= n) continue;
+      const u32 t = t0 + j0 + j, h = tok_hash(tag, t);
+      if (v[j].x == tag && v[j].y == t && v[j].z == h && v[j].w == ~h) {
+        cs += h;
+      } else {
+        if (!nbad) first_bad = (u64)v[j].x | ((u64)v[j].y << 32);
+        ++nbad;
+      }
+    }
+  }
+}
+
+// A step's check: begin issues the loads of the first pass, so that they arrive
+// with what the caller does before finish.
+struct Drain {
+  u64 rem;  // the lanes whose pages no pass has taken
+  bool share;
+  DrainPass d;
+};
+__device__ __forceinline__ Drain drain_begin(bool drains, u32 me, const uint4* pg, u32 tag, u32 drain, u32 tok) {
+  Drain x;
+  const u64 D = __ballot(drains);
+  x.share = (u32)__builtin_popcountll(D) <= DRAIN_SHARED;
+  x.rem = x.share ? D : 0;
+  x.d = drain_load(x.rem, me, pg, tag, drain, tok);
+  return x;
+}
+__device__ __forceinline__ void drain_finish(Drain& x, bool drains, u32 me, const uint4* pg, u32 tag, u32 drain,
+                                             u32 tok, u32& cs, u32& nbad, u64& first_bad) {
+  if (!x.share && drains) drain_own(pg, tag, drain, tok, cs, nbad, first_bad);
+  while (x.d.any) {
+    drain_check(x.d, me, cs, nbad, first_bad);
+    x.d = drain_load(x.rem, me, pg, tag, drain, tok);
+  }
+}
+
+// One step's check on pages in a caller's buffer (one page per lane).
+__global__ void __launch_bounds__(64) drain_check_k(const uint4* pages, const u32* tag, const u32* drain,
+                                                    const u32* tok, const u32* drains, u32* cs, u32* nbad,
+                                                    u64* first_bad) {
+  const u32 me = threadIdx.x;
+  const uint4* pg = pages + me * SRV_TOK_PER_PAGE;
+  u32 c = cs[me], b = nbad[me];
+  u64 f = first_bad[me];
+  Drain x = drain_begin(drains[me] != 0, me, pg, tag[me], drain[me], tok[me]);
+  drain_finish(x, drains[me] != 0, me, pg, tag[me], drain[me], tok[me], c, b, f);
+  cs[me] = c;
+  nbad[me] = b;
+  first_bad[me] = f;
 }
 
 __global__ void __launch_bounds__(256) srv_loop_k(SrvArgs a) {
@@ -1344,20 +1427,15 @@ __global__ void __launch_bounds__(256) srv_loop_k(SrvArgs a) {
         ++my_stalls;
       }
     }
-    // ---- one step per live sequence.  The lanes that drain a page share its
-    // check with the whole wave: one token per lane, four pages at a time, one
-    // coalesced load each time.  In most iterations only some of the 64 lanes
-    // drain, and a lane that checked its own page made the wave run 16 hashes
-    // one after another (and hold 16 tokens in registers: 153 -> 81 VGPRs).
-    // The first four pages are loaded before the mallocs and arrive with them.
-    // Bound by the round trips of one malloc and one free per iteration, with
-    // one wave per SIMD: 20 000 requests, median 256 tokens, 8.0 -> 7.2 ms.
+    // ---- one step per live sequence.  The first pages to be checked are loaded
+    // before the mallocs and arrive with them.  Bound by the round trips of one
+    // malloc and one free per iteration, with one wave per SIMD: 20 000
+    // requests, median 256 tokens, 8.0 -> 7.2 ms with the shared check.
     bool sampled = false, finished = false;
     u32 lat = 0;
     const bool drains = req != SRV_NONE && draining && drain < np;
     const bool ends = req != SRV_NONE && draining && drain + 1 >= np;  // after this step
-    u64 rem = __ballot(drains);
-    DrainPass d = drain_load(rem, me, next_pg, tag, drain, tok);
+    Drain chk = drain_begin(drains, me, next_pg, tag, drain, tok);
     if (req != SRV_NONE && !draining) {
       if (tok % SRV_TOK_PER_PAGE == 0) {
         const u32 pi = tok / SRV_TOK_PER_PAGE;
@@ -1391,10 +1469,7 @@ __global__ void __launch_bounds__(256) srv_loop_k(SrvArgs a) {
         drain = 0;
       }
     }
-    while (d.any) {
-      drain_check(d, me, cs, nbad, first_bad);
-      d = drain_load(rem, me, next_pg, tag, drain, tok);
-    }
+    drain_finish(chk, drains, me, next_pg, tag, drain, tok, cs, nbad, first_bad);
     if (drains) {
       hafree((void*)next_pg);
       ++drain;
@@ -2947,6 +3022,34 @@ int ha_run_graphs(const ha_graph_args* a, const uint32_t* nnodes, ha_graph_resul
   res->plain_ms = a->run_plain ? best_plain : 0;
   res->batch_ms = a->run_batch ? best_batch : 0;
   res->plain_launches = (int32_t)(2 * chunks.size());
+  return HA_OK;
+}
+
+int ha_check_pages(const uint32_t* pages, const uint32_t* tag, const uint32_t* drain, const uint32_t* tok,
+                   const uint32_t* drains, uint32_t* checksum, uint32_t* bad, uint64_t* bad_first) {
+  if (!pages || !tag || !drain || !tok || !drains || !checksum || !bad || !bad_first)
+    return hfail(HA_E_INVALID, "null argument");
+  for (int i = 0; i < 64; ++i)
+    if (drains[i] && (tok[i] > 32768 || drain[i] >= 32768 / SRV_TOK_PER_PAGE ||
+                      tok[i] <= drain[i] * SRV_TOK_PER_PAGE))
+      return hfail(HA_E_INVALID, "a drained page must hold one of the sequence's tokens");
+  DBuf dp, du, df;  // du: tag, drain, tok, drains, checksum, bad
+  HH(dp.alloc(64 * SRV_PAGE_BYTES));
+  HH(du.alloc(6 * 64 * 4));
+  HH(df.alloc(64 * 8));
+  u32* u = (u32*)du.p;
+  const uint32_t* in[6] = {tag, drain, tok, drains, checksum, bad};
+  for (int i = 0; i < 6; ++i) HH(hipMemcpy(u + 64 * i, in[i], 64 * 4, hipMemcpyHostToDevice));
+  HH(hipMemcpy(dp.p, pages, 64 * SRV_PAGE_BYTES, hipMemcpyHostToDevice));
+  HH(hipMemcpy(df.p, bad_first, 64 * 8, hipMemcpyHostToDevice));
+  Stream s;
+  HH(s.create());
+  drain_check_k<<<1, 64, 0, s.s>>>((const uint4*)dp.p, u, u + 64, u + 128, u + 192, u + 256, u + 320, (u64*)df.p);
+  HH(hipGetLastError());
+  HH(hipStreamSynchronize(s.s));
+  HH(hipMemcpy(checksum, u + 256, 64 * 4, hipMemcpyDeviceToHost));
+  HH(hipMemcpy(bad, u + 320, 64 * 4, hipMemcpyDeviceToHost));
+  HH(hipMemcpy(bad_first, df.p, 64 * 8, hipMemcpyDeviceToHost));
   return HA_OK;
 }
 

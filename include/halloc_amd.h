@@ -288,6 +288,14 @@ typedef struct ha_serve_result {
   uint32_t completed, admitted, clock_khz, pad;
 } ha_serve_result;
 int ha_run_serve(const ha_serve_io *io, ha_serve_result *res);
+/* The serving loop's check of drained pages, one step of one wave, on pages the
+   caller prepared (tests give it damaged ones).  Arrays of 64, entry l for lane
+   l: pages (64 words each: 16 tokens {tag, t, hash, ~hash}), the sequence's tag,
+   the page's index, the sequence's token count, and whether the lane drains.
+   The step adds to checksum and bad and sets bad_first (words 0 and 1 of the
+   sequence's first damaged token) where bad was 0. */
+int ha_check_pages(const uint32_t *pages, const uint32_t *tag, const uint32_t *drain, const uint32_t *tok,
+                   const uint32_t *drains, uint32_t *checksum, uint32_t *bad, uint64_t *bad_first);
 
 /* The reference test programs' kernels (tst/corr/checkptr, tst/corr/prob-checkptr,
    tst/perf/throughput, tst/perf/priv-throughput) for the option set of

@@ -183,6 +183,49 @@ def test_pages_drained_together(heap, nreq, length):
         assert r["pages"] == int(pages_for(ln).sum())
 
 
+@pytest.mark.parametrize("lanes", [1, 3, 4, 5, 7, 8, 9, 12, 16, 33, 63, 64])
+def test_damaged_pages_are_charged_to_their_lanes(heap, lanes):
+    # the wave's check and each lane's own, on pages with damaged tokens: up to
+    # and above the number of lanes from which each checks its own page, passes
+    # of four pages with one to four owners, part-filled pages (what follows
+    # their tokens is never looked at), lanes that already found damage
+    from tests.helpers import _hash3
+    print(f"[gpu] damaged pages lanes={lanes}", flush=True)
+    rng = np.random.default_rng(lanes)
+    some = 0
+    for rate in (0.0, 0.05, 0.5, 1.0):
+        tag = rng.integers(0, 1 << 32, 64, dtype=np.uint64).astype(np.uint32)
+        page = rng.integers(0, 2048, 64).astype(np.uint32)
+        n = np.where(rng.random(64) < 0.5, 16, rng.integers(1, 17, 64)).astype(np.int64)
+        drains = np.zeros(64, np.uint32)
+        drains[rng.permutation(64)[:lanes]] = 1
+        t = page[:, None] * np.uint32(16) + np.arange(16, dtype=np.uint32)
+        h = _hash3(np.repeat(tag, 16), t.ravel(), np.uint32(0x5E7A11C3)).reshape(64, 16)
+        pages = np.stack([np.repeat(tag[:, None], 16, 1), t, h, ~h], axis=-1)
+        used = np.arange(16) < n[:, None]
+        hurt = (rng.random((64, 16)) < rate) & used
+        l, j = np.nonzero(hurt)
+        pages[l, j, rng.integers(0, 4, l.size)] ^= np.uint32(1) << rng.integers(0, 32, l.size).astype(np.uint32)
+        pages[~used] = rng.integers(0, 1 << 32, (int((~used).sum()), 4), dtype=np.uint64).astype(np.uint32)
+        cs0 = rng.integers(0, 1 << 32, 64, dtype=np.uint64).astype(np.uint32)
+        nb0 = rng.choice([0, 0, 3], 64).astype(np.uint32)
+        bf0 = rng.integers(0, 1 << 62, 64, dtype=np.uint64)
+        cs, nb, bf = H.Halloc.check_pages(pages, tag, page, page * 16 + n, drains, cs0, nb0, bf0)
+        for i in range(64):
+            bad = np.nonzero(hurt[i])[0] if drains[i] else np.zeros(0, int)
+            good = h[i][used[i] & ~hurt[i]] if drains[i] else h[i][:0]
+            assert cs[i] == (int(cs0[i]) + int(good.astype(np.uint64).sum())) & 0xFFFFFFFF
+            assert nb[i] == nb0[i] + bad.size
+            first = bf0[i]
+            if bad.size and not nb0[i]:
+                first = int(pages[i, bad[0], 0]) | int(pages[i, bad[0], 1]) << 32
+            assert bf[i] == first
+            some += bad.size
+    assert some > 0
+    with pytest.raises(H.HallocError):
+        H.Halloc.check_pages(pages, tag, page, page * 16, np.ones(64), cs0, nb0, bf0)
+
+
 @pytest.mark.parametrize("nthreads", [1, 4])
 def test_buffers_kept_between_calls(heap, nthreads):
     # calls of changing sizes, from several threads, with a refused call between:
