@@ -2447,9 +2447,20 @@ int ha_run_test(const ha_test_opts* a, ha_test_result* r) {
   };
   const unsigned grid = (n + (u32)a->bs - 1) / (u32)a->bs;
   unsigned long long* st = (unsigned long long*)ds.p;
-  // queued behind the launch it checks; its counts are read once, at the end
+  // Queued behind the launch it checks; its counts are read once, at the end.
+  // Its grid is a whole number of rounds over the compute units, so that the
+  // launches that are timed are dealt out as if it were not there.  With the
+  // grid of those launches it moved the next one's blocks to other compute
+  // units, and so to other head sets, than the free before it: filling 40% of
+  // 512 MiB took 900-965 us with 1536 B blocks, 750-790 with 2048 B and 735-770
+  // with 3072 B, against 855, 728 and 690 now; the same grid with an empty
+  // kernel cost as much.
+  int dev = 0, ncu = 0;
+  HH(hipGetDevice(&dev));
+  HH(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  const unsigned cu = ncu > 0 ? (unsigned)ncu : 1u, cgrid = (grid + cu - 1) / cu * cu;
   auto check_nz = [&](bool with_ctrs, int t) -> int {
-    t_check_nz_k<<<grid, a->bs, 0, s.s>>>(o, (void* const*)dp.p, with_ctrs ? (const u32*)dc.p : nullptr, (u32)t, st + 3);
+    t_check_nz_k<<<cgrid, a->bs, 0, s.s>>>(o, (void* const*)dp.p, with_ctrs ? (const u32*)dc.p : nullptr, (u32)t, st + 3);
     HH(hipGetLastError());
     return HA_OK;
   };

@@ -45,6 +45,23 @@ def test_null_check_counts_the_nulls_held(heap, test, n, bs, nallocs, period, gr
     assert r["mallocs"] == r["frees"]
 
 
+@pytest.mark.parametrize("test", ["phase-throughput", "phase-latency"])
+@pytest.mark.parametrize("n,bs,period,group", [(24000, 100, 0, 0), (23999, 256, 0, 0), (48000, 64, 1, 5)])
+def test_null_check_names_the_first_failing_try(heap, test, n, bs, period, group):
+    # half of the threads without a block allocate at each even try and nothing
+    # is freed: 12 000 blocks of 3072 B fit a 48 MiB slab heap, 18 000 do not, so
+    # the NULLs begin at try 2, and every later check counts all that are held
+    print(f"[gpu] first failing try {test} n={n} bs={bs} period={period}", flush=True)
+    opts = H.HallocOpts(memory=64 << 20, sb_sz_sh=21, nheads=1)
+    for ntries in range(1, 5):
+        heap(opts)  # starts an empty heap
+        r = run(test, n, bs, 3072, ntries=ntries, period=period, group=group, probabs=((0.5, 0.0), (0.0, 0.0)))
+        assert (r["nulls"] > 0) == (ntries > 2)
+        assert r["failed_try"] == (2 if ntries > 2 else -1)
+        assert r["checks_failed"] == max(ntries - 2, 0) * r["nulls"]  # try 3 changes nothing
+        assert r["mallocs"] == r["frees"]
+
+
 # lanes that take part in a batched call: a wave whose low lanes are inactive
 # (the per-round values must not be kept in lanes 0..15), fewer lanes than
 # rounds, every other lane, one lane
