@@ -281,6 +281,41 @@ def test_buffers_kept_between_calls(heap, nthreads):
         H.Halloc.shutdown()
 
 
+def test_long_lists_from_several_threads(heap):
+    # lists that the device checks, in buffers that calls of other lengths and
+    # threads gave back: good orders are taken, others refused
+    import threading
+
+    print("[gpu] long lists from several threads", flush=True)
+    heap(H.HallocOpts(memory=1 << 30, sb_sz_sh=22))
+    wrong = []
+
+    def calls(t):
+        try:
+            rng = np.random.default_rng(t)
+            for n in (1 << 17, 70, 150001, 1 << 17, 200003):
+                sizes = (rng.integers(0, 3, (1, n)) * 16).astype(np.uint32)
+                order = rng.permutation(n).astype(np.uint32)
+                for _ in range(2):
+                    r = H.Halloc.run_lists(sizes, order)
+                    assert r["requests"] == np.count_nonzero(sizes) and r["nulls"] == 0 and r["errors"] == 0
+                    bad = order.copy()
+                    bad[rng.integers(0, n)] = rng.choice([n, order[0], order[n - 1]])
+                    if (np.sort(bad) != np.arange(n)).any():
+                        with pytest.raises(H.HallocError, match="permutation"):
+                            H.Halloc.run_lists(sizes, bad)
+        except BaseException as e:  # reported below: a thread's own failure would be lost
+            wrong.append(repr(e))
+
+    ths = [threading.Thread(target=calls, args=(t,)) for t in range(4)]
+    for th in ths:
+        th.start()
+    for th in ths:
+        th.join()
+    assert not wrong
+    assert H.Halloc.free_bytes() == H.Halloc.geometry()["arena_bytes"]
+
+
 @pytest.mark.parametrize("n,per", [(1, 1), ((1 << 17) - 1, 1), (1 << 16, 2), (43691, 3), (1 << 17, 1), (100003, 7)])
 def test_list_orders_checked(heap, n, per):
     # below, at and above the length from which the device checks the order and
