@@ -651,8 +651,8 @@ HA_DEV u32 mod_chunks(const SizeInfo& s, u64 x) {
 // marked is below the busy threshold and is probed on, whichever it is.
 // Loading the counter at every check put loads and atomics on one line, and
 // where the L2 caches a line that others add to, each waits for the other:
-// 64 words hot at once, an atomic alone took 22 ns a word, with a load beside
-// it 213 ns.  2^20 threads of 8..256 B on 512 MiB, where two counters a class
+// 64 words hot at once, an atomic alone takes 22 ns a word, with a load beside
+// it 220 ns.  2^20 threads of 8..256 B on 512 MiB, where two counters a class
 // serve the whole chip, took 3.5 ms a launch of four rounds and take 1.5 ms
 // with the mark.
 HA_DEV u64 probe_run(const Params& P_, const SizeInfo& s, u32 hsb, u32 limit, u32 old, u64 P, u32 me, u32& itry, u32& my_ich,
